@@ -297,9 +297,10 @@ int spbp_set_symmetries(spbp_ctx* ctx, int nsym, const double* angles_deg);
 /* Plan = insertion strategy (SPBP_STRAT_DIRECT / _BRICK / _GATHER), brick shape
  * (0: 16x16x8, 1: 16x8x8, 2: 8x8x8, 3: 16x12x8, 4: 16x16x10, 5: 16x16x12,
  * 6: 16x16x13 voxels = the LDS bin, every sample evaluated in each bin its
- * taps reach; 7, the default: owner-computes bins, a 16x16x13 LDS region
- * around a 12x12x9 core, each sample evaluated only in the bin whose core
- * holds its nearest voxel) and projections per
+ * taps reach; 7, the default: owner-computes bins, each sample evaluated only
+ * in the bin that holds its unit cell, a 12x12x12 LDS region around 9x9x9
+ * cells -- or, in launches of fewer than 2 NX sections per half, its nearest
+ * voxel, a 16x16x13 region around a 12x12x9 core) and projections per
  * brick work item (default 128; a launch of fewer than 8 x that many
  * sections halves it, down to 16, so its busiest bricks still split).  spbp_tune times every plan on a sample of
  * up to 1024 of the given images (into scratch grids: the accumulators are

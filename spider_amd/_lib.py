@@ -68,7 +68,8 @@ class FinalJob(C.Structure):
 
 
 SHAPES = [(16, 16, 8), (16, 8, 8), (8, 8, 8), (16, 12, 8), (16, 16, 10), (16, 16, 12), (16, 16, 13), (16, 16, 13)]
-# owner-computes bricks (SHAPES gives the LDS region; each sample is evaluated in one brick only)
+# owner-computes bricks (SHAPES gives the LDS region; each sample is evaluated in one brick only).  The region of plan 7
+# is that of its launches with few sections; the others take 12x12x12 regions around 9x9x9 unit cells.
 SHAPE_OWN = [False] * 7 + [True]
 TUNE_C = [16, 32, 64, 128]
 

@@ -128,7 +128,8 @@ struct BrickGrid {
     int bx, by, bz;      // brick edge (voxels); the core's with owner-computes bricks
     int nbx, nby, nbz;   // bricks per axis
     int nb;              // nbx * nby * nbz
-    int own;             // owner-computes bricks (LDS region = core + 2 per side)
+    int own;             // owner-computes bricks: 1 by nearest voxel (LDS region = core + 2 per side), 2 by unit
+                         // cell (region = cells + 1 before and 2 after; insert_cells.hpp)
 };
 
 __device__ inline void brick_origin(const BrickGrid& bg, int b, int nx, int& x0, int& y0, int& z0) {
@@ -180,9 +181,10 @@ __host__ __device__ __forceinline__ SuperBrick superbrick(const BrickGrid& bg, i
         g.b[d] = (i < bg.nbx && j < bg.nby && k < bg.nbz) ? i + bg.nbx * (j + bg.nby * k) : -1;
         // the member's expanded box and its disk condition
         const int x0 = i * bg.bx, y0 = -nx + 1 + j * bg.by, z0 = -nx + 1 + k * bg.bz;
-        const float m = bg.own ? (x0 == 0 ? 2.52f : 0.52f) : BRICK_MARGIN;
+        const float m = bg.own == 2 ? 0.52f : bg.own ? (x0 == 0 ? 2.52f : 0.52f) : BRICK_MARGIN;
+        const float sh = bg.own == 2 ? 0.5f : 0.0f;   // cells [x, x + 1): the box lies half a voxel further on
         const float hx = 0.5f * (bg.bx - 1) + m, hy = 0.5f * (bg.by - 1) + m, hz = 0.5f * (bg.bz - 1) + m;
-        const float cx = x0 + 0.5f * (bg.bx - 1), cy = y0 + 0.5f * (bg.by - 1), cz = z0 + 0.5f * (bg.bz - 1);
+        const float cx = x0 + 0.5f * (bg.bx - 1) + sh, cy = y0 + 0.5f * (bg.by - 1) + sh, cz = z0 + 0.5f * (bg.bz - 1) + sh;
         const float qx = fmaxf(fabsf(cx) - hx, 0.f), qy = fmaxf(fabsf(cy) - hy, 0.f), qz = fmaxf(fabsf(cz) - hz, 0.f);
         if (!(qx * qx + qy * qy + qz * qz <= r * r)) g.b[d] = -1;
         g.mc[d][0] = cx;
@@ -193,7 +195,8 @@ __host__ __device__ __forceinline__ SuperBrick superbrick(const BrickGrid& bg, i
         g.mh[d][2] = hz;
     }
     const int i1 = min(2 * si + 1, bg.nbx - 1), j1 = min(2 * sj + 1, bg.nby - 1), k1 = min(2 * sk + 1, bg.nbz - 1);
-    const float m = (bg.own ? (si == 0 ? 2.52f : 0.52f) : BRICK_MARGIN) + 0.05f;
+    // cells: the group's box from -0.57 to +1.07 holds the members' [-0.02, +1.02]
+    const float m = (bg.own == 2 ? 1.02f : bg.own ? (si == 0 ? 2.52f : 0.52f) : BRICK_MARGIN) + 0.05f;
     const float xlo = 2 * si * bg.bx - m, xhi = i1 * bg.bx + bg.bx - 1 + m;
     const float ylo = -nx + 1 + 2 * sj * bg.by - m, yhi = -nx + 1 + j1 * bg.by + bg.by - 1 + m;
     const float zlo = -nx + 1 + 2 * sk * bg.bz - m, zhi = -nx + 1 + k1 * bg.bz + bg.bz - 1 + m;

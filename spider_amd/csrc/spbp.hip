@@ -47,6 +47,7 @@
 #include "finalize.hpp"
 #include "hostmath.hpp"
 #include "insert.hpp"
+#include "insert_cells.hpp"
 #include "insert_gather.hpp"
 #include "project.hpp"
 #include "resolve.hpp"
@@ -60,10 +61,13 @@ constexpr int ERR_LEN = 512;
 thread_local char g_last_error[ERR_LEN] = {0};
 // brick shapes of the LDS-binned strategy (voxels; 3 x 8 B per voxel in LDS)
 // {x, y, z, owner-computes}; for owner-computes bricks the LDS region, whose
-// core (each sample's owner) is 4 voxels shorter per axis
+// core (each sample's owner) is 4 voxels shorter per axis by nearest voxel
+// (1), 3 by unit cell (2)
 constexpr int NSHAPES = 8;
-constexpr int SHAPES[NSHAPES][4] = {{16, 16, 8, 0},  {16, 8, 8, 0},   {8, 8, 8, 0},    {16, 12, 8, 0},
-                                    {16, 16, 10, 0}, {16, 16, 12, 0}, {16, 16, 13, 0}, {16, 16, 13, 1}};
+constexpr int SHAPE_CELLS = 7, SHAPE_OWN = 8;   // unit cells; nearest voxel (not a plan of its own)
+constexpr int SHAPES[NSHAPES + 1][4] = {{16, 16, 8, 0},  {16, 8, 8, 0},   {8, 8, 8, 0},
+                                        {16, 12, 8, 0},  {16, 16, 10, 0}, {16, 16, 12, 0},
+                                        {16, 16, 13, 0}, {12, 12, 12, 2}, {16, 16, 13, 1}};
 // brick workgroups: 16x16x10, 16x16x12 and 16x16x13 (61.7, 73.8 and 80.2 KB of
 // LDS) run two 512-thread groups per CU; the others four (three for 16x16x8)
 // 256-thread groups.  The FP64-geometry instantiations need more VGPRs than
@@ -188,7 +192,8 @@ struct spbp_ctx {
     int jobs_cap = 0;
     hipEvent_t jobs_evt = nullptr;
     int ncu = 256;
-    BrickGrid bg{};
+    BrickGrid bg{};         // the shape's brick grid
+    BrickGrid bgo{};        // unit-cell shape: the nearest-voxel bricks of launches with few sections (nb 0 otherwise)
     int* bcnt = nullptr;    // [2 nb] hits per (brick, half)
     int* boff = nullptr;    // [2 nb + 1] list offsets
     int* bioff = nullptr;   // [2 nb + 1] work-item offsets
@@ -322,7 +327,7 @@ int refuse_captured(spbp_ctx* c, const char* what) {
 // contexts have no shared-evaluation 16x16x12 / 16x16x13 kernels: 16x16x10).
 BrickGrid grid_of_shape(int nx, int flags, int& shape) {
     if ((flags & SPBP_GEOM_F64) && (shape == 5 || shape == 6)) shape = 4;
-    const int own = SHAPES[shape][3], halo = own ? 4 : 0;
+    const int own = SHAPES[shape][3], halo = own == 2 ? 3 : own ? 4 : 0;
     const int bx = SHAPES[shape][0] - halo, by = SHAPES[shape][1] - halo, bz = SHAPES[shape][2] - halo;
     BrickGrid g;
     g.bx = bx;
@@ -355,9 +360,22 @@ int configure_bricks(spbp_ctx* c, int shape) {
     HIPCHK(c, dmalloc(&c->bcur, nk * sizeof(int)));
     HIPCHK(c, dmalloc(&c->bscan, ((nk + 1023) / 1024 + 1) * sizeof(int2)));
     c->bg = g;
+    c->bgo = BrickGrid{};
+    if (shape == SHAPE_CELLS) {   // never more bricks than the unit cells' (whose edges are shorter): the same arrays
+        int so = SHAPE_OWN;
+        c->bgo = grid_of_shape(c->nx, c->flags, so);
+    }
     c->shape = shape;
     return SPBP_OK;
 }
+
+// Launches with few sections take the nearest-voxel bricks: a unit-cell work
+// item costs some 25 us however few sections it holds, which 2 NX sections
+// per half repay (insertion, nearest voxel / unit cells, us: 128^2, 128
+// sections 377 / 449, 256 505 / 500, 512 783 / 626, 2048 2574 / 1716; 256^2,
+// 256 2431 / 2972, 512 3273 / 3380, 1024 5243 / 4309; 64^2, 128 123 / 125,
+// 256 172 / 138).
+bool few_sections(const spbp_ctx* c, int nsec) { return c->bgo.nb > 0 && nsec < 2 * c->nx * c->nvol; }
 
 // Projection lists for chunks of up to B projections.  The capacity is
 // committed only once both arrays exist.
@@ -581,18 +599,24 @@ struct Targets {
     float2* X0; float* W0; float2* X1; float* W1; float* Wc0; float* Wc1;
 };
 
+// The most sections a work item of the context's brick kernel may hold.
+int max_item(const spbp_ctx* c, bool few) {
+    if (c->shape != SHAPE_CELLS || few) return 128;
+    return (c->flags & SPBP_GEOM_F64) ? CELL_SECS64 : CELL_SECS;
+}
+
 // Projections per work item for a launch of nsec sections: the plan's C,
 // halved while the launch holds fewer than 8 x C sections (down to 16), so
 // the bricks every plane crosses still split into several items.  Measured at
 // 128^2 into 256^3 with 256-section launches: 294k proj/s with 16 or 32 per
 // item, 212k with 128.
-int item_proj(int C, int nsec) {
+int item_proj(int C, int nsec, int limit) {
     int k = C;
     while (k > 16 && 8 * k > nsec) k >>= 1;
-    return k;
+    return std::min(k, limit);
 }
 
-BrickJob brick_job(const spbp_ctx* c, int img0, const Geom* geom_d, int nsec, const Targets& t) {
+BrickJob brick_job(const spbp_ctx* c, int img0, const Geom* geom_d, int nsec, const Targets& t, bool few) {
     BrickJob j;
     j.wscale = WSCALE;
     j.spec = c->spec;
@@ -603,8 +627,8 @@ BrickJob brick_job(const spbp_ctx* c, int img0, const Geom* geom_d, int nsec, co
     j.fltb = c->fltb;
     j.nx = c->nx;
     j.N = c->N;
-    j.C = item_proj(c->C, nsec);
-    j.bg = c->bg;
+    j.C = item_proj(c->C, nsec, max_item(c, few));
+    j.bg = few ? c->bgo : c->bg;
     j.cnt = c->bcnt;
     j.off = c->boff;
     j.item_off = c->bioff;
@@ -614,12 +638,13 @@ BrickJob brick_job(const spbp_ctx* c, int img0, const Geom* geom_d, int nsec, co
     return j;
 }
 
-unsigned brick_grid(const spbp_ctx* c) {
+unsigned brick_grid(const spbp_ctx* c, bool few) {
     // workgroups resident per CU: the 512-thread shapes (16x16x10, 16x16x12,
     // 16x16x13: 61.7, 73.8 and 80.2 KB of LDS with weights) run two per CU,
     // 16x16x8 (49.2 KB) three, the other 256-thread shapes four (VGPR-bound:
     // 4 waves per SIMD); the FP64-geometry instantiations need ~150-170
     // VGPRs: one 512-thread group or three 256-thread groups per CU
+    if (c->shape == SHAPE_CELLS && !few) return (unsigned)c->ncu;
     if (c->shape >= 4) return (unsigned)c->ncu * ((c->flags & SPBP_GEOM_F64) ? 1u : 2u);
     return (unsigned)c->ncu * ((c->shape == 0 || (c->flags & SPBP_GEOM_F64)) ? 3u : 4u);   // 16x12x8: 36.9 KB, 4 fit
 }
@@ -630,13 +655,19 @@ void launch_shape(bool wgt, unsigned grid, const BrickJob* table_d, int n, int* 
     else insert_brick_kernel<BX, BY, BZ, P, NT, OWN, false><<<grid, NT, 0, st>>>(table_d, n, counter);
 }
 
+template <typename P>
+void launch_cells(bool wgt, unsigned grid, const BrickJob* table_d, int n, int* counter, hipStream_t st) {
+    if (wgt) insert_cells_kernel<CELL_EDGE, CELL_EDGE, CELL_EDGE, P, CELL_NT, true><<<grid, CELL_NT, 0, st>>>(table_d, n, counter);
+    else insert_cells_kernel<CELL_EDGE, CELL_EDGE, CELL_EDGE, P, CELL_NT, false><<<grid, CELL_NT, 0, st>>>(table_d, n, counter);
+}
+
 // One persistent brick-kernel launch over the device job table table_d[0..n),
 // all jobs with c's brick shape; `counter` (the queue head) must be zero on st.
 // wgt false: no job accumulates weights (W0 and W1 null in every job).
-int launch_bricks_dev(spbp_ctx* c, const BrickJob* table_d, int n, int* counter, hipStream_t st, bool wgt = true) {
-    const unsigned grid = brick_grid(c);
+int launch_bricks_dev(spbp_ctx* c, const BrickJob* table_d, int n, int* counter, hipStream_t st, bool wgt, bool few) {
+    const unsigned grid = brick_grid(c, few);
     const bool f64 = (c->flags & SPBP_GEOM_F64) != 0;
-    switch (c->shape * 2 + (f64 ? 1 : 0)) {
+    switch ((few ? SHAPE_OWN : c->shape) * 2 + (f64 ? 1 : 0)) {
         case 0: launch_shape<16, 16, 8, float>(wgt, grid, table_d, n, counter, st); break;
         case 1: launch_shape<16, 16, 8, double>(wgt, grid, table_d, n, counter, st); break;
         case 2: launch_shape<16, 8, 8, float>(wgt, grid, table_d, n, counter, st); break;
@@ -649,8 +680,10 @@ int launch_bricks_dev(spbp_ctx* c, const BrickJob* table_d, int n, int* counter,
         case 9: launch_shape<16, 16, 10, double, 2 * TPB>(wgt, grid, table_d, n, counter, st); break;
         case 10: launch_shape<16, 16, 12, float, 2 * TPB>(wgt, grid, table_d, n, counter, st); break;
         case 12: launch_shape<16, 16, 13, float, 2 * TPB>(wgt, grid, table_d, n, counter, st); break;
-        case 14: launch_shape<16, 16, 13, float, 2 * TPB, true>(wgt, grid, table_d, n, counter, st); break;
-        case 15: launch_shape<16, 16, 13, double, 2 * TPB, true>(wgt, grid, table_d, n, counter, st); break;
+        case 14: launch_cells<float>(wgt, grid, table_d, n, counter, st); break;
+        case 15: launch_cells<double>(wgt, grid, table_d, n, counter, st); break;
+        case 16: launch_shape<16, 16, 13, float, 2 * TPB, true>(wgt, grid, table_d, n, counter, st); break;
+        case 17: launch_shape<16, 16, 13, double, 2 * TPB, true>(wgt, grid, table_d, n, counter, st); break;
         default: return fail(c, SPBP_ERR_ARG, "brick shape %d has no FP64-geometry kernel", c->shape);
     }
     HIPCHK(c, hipGetLastError());
@@ -658,7 +691,7 @@ int launch_bricks_dev(spbp_ctx* c, const BrickJob* table_d, int n, int* counter,
 }
 
 // Same with a host job table, staged through c's pinned buffer.
-int launch_bricks(spbp_ctx* c, const BrickJob* jh, int n, int* counter, hipStream_t st, bool wgt = true) {
+int launch_bricks(spbp_ctx* c, const BrickJob* jh, int n, int* counter, hipStream_t st, bool wgt, bool few) {
     if (n < 1 || n > MAX_JOBS) return fail(c, SPBP_ERR_ARG, "%d jobs in one launch (1..%d)", n, MAX_JOBS);
     if (c->jobs_cap < n) {
         if (c->jobs_h) { (void)hipEventSynchronize(c->jobs_evt); (void)hipHostFree(c->jobs_h); c->jobs_h = nullptr; }
@@ -672,27 +705,28 @@ int launch_bricks(spbp_ctx* c, const BrickJob* jh, int n, int* counter, hipStrea
     std::memcpy(c->jobs_h, jh, n * sizeof(BrickJob));
     HIPCHK(c, hipMemcpyAsync(c->jobs_d, c->jobs_h, n * sizeof(BrickJob), hipMemcpyHostToDevice, st));
     HIPCHK(c, hipEventRecord(c->jobs_evt, st));
-    return launch_bricks_dev(c, c->jobs_d, n, counter, st, wgt);
+    return launch_bricks_dev(c, c->jobs_d, n, counter, st, wgt, few);
 }
 
 // Per-(brick, half) projection lists of b projections (geometry at geom_d);
 // also zeroes c's queue head.
-int build_lists(spbp_ctx* c, const Geom* geom_d, int b, hipStream_t st) {
-    if (c->bg.nb <= 0 || !c->bcnt || !c->blist || !c->bikey || c->blist_cap < (size_t)b * c->bg.nb || !c->bpln ||
+int build_lists(spbp_ctx* c, const Geom* geom_d, int b, hipStream_t st, bool few) {
+    const BrickGrid& bg = few ? c->bgo : c->bg;
+    if (c->bg.nb <= 0 || bg.nb > c->bg.nb || !c->bcnt || !c->blist || !c->bikey || c->blist_cap < (size_t)b * c->bg.nb || !c->bpln ||
         c->bpln_cap < (size_t)b)
         return fail(c, SPBP_ERR_ARG, "brick lists not allocated for %d sections", b);
-    const int nkeys = 2 * c->bg.nb;
-    const int nsb = ((c->bg.nbx + 1) / 2) * ((c->bg.nby + 1) / 2) * ((c->bg.nbz + 1) / 2);   // superbricks
+    const int nkeys = 2 * bg.nb;
+    const int nsb = ((bg.nbx + 1) / 2) * ((bg.nby + 1) / 2) * ((bg.nbz + 1) / 2);   // superbricks
     const dim3 lgrid(nsb, (b + 1023) / 1024);
     Timed tm(c, SPBP_K_BIN, b, st);
     fill((float*)c->bcnt, nkeys, 0.0f, st);   // zero bits
     plane_pack_kernel<<<nblocks(b), TPB, 0, st>>>(geom_d, b, c->bpln);
-    brick_count_kernel<<<lgrid, TPB, 0, st>>>(c->bpln, b, c->bg, c->nx, c->bcnt);
+    brick_count_kernel<<<lgrid, TPB, 0, st>>>(c->bpln, b, bg, c->nx, c->bcnt);
     const int kb = (nkeys + 1023) / 1024;
-    key_scan_blocks_kernel<<<kb, 1024, 0, st>>>(c->bcnt, nkeys, item_proj(c->C, b), c->boff, c->bioff, c->bscan);
+    key_scan_blocks_kernel<<<kb, 1024, 0, st>>>(c->bcnt, nkeys, item_proj(c->C, b, max_item(c, few)), c->boff, c->bioff, c->bscan);
     key_scan_sums_kernel<<<1, 1024, 0, st>>>(c->bscan, kb, nkeys, c->boff, c->bioff, c->bnext);
     key_scan_add_kernel<<<kb, 1024, 0, st>>>(nkeys, c->bscan, c->boff, c->bioff, c->bcur);
-    brick_fill_kernel<<<lgrid, TPB, 0, st>>>(c->bpln, b, c->bg, c->nx, c->boff, c->bcur, c->blist);
+    brick_fill_kernel<<<lgrid, TPB, 0, st>>>(c->bpln, b, bg, c->nx, c->boff, c->bcur, c->blist);
     brick_itemkey_kernel<<<nblocks(nkeys), TPB, 0, st>>>(c->bioff, nkeys, c->bikey);
     HIPCHK(c, hipGetLastError());
     return SPBP_OK;
@@ -750,11 +784,12 @@ int run_insert(spbp_ctx* c, int img0, const Geom* geom_d, int ng, const Targets&
     if (!c->spec || !c->vmax || ng > c->fwd_batch * c->nsym)
         return fail(c, SPBP_ERR_ARG, "chunk buffers not allocated for %d sections", ng);
     if (own_kernel(c)) return launch_own(c, img0, geom_d, ng, t, st, units);
-    int rc = build_lists(c, geom_d, ng, st);
+    const bool few = few_sections(c, ng);
+    int rc = build_lists(c, geom_d, ng, st, few);
     if (rc) return rc;
-    const BrickJob job = brick_job(c, img0, geom_d, ng, t);
+    const BrickJob job = brick_job(c, img0, geom_d, ng, t, few);
     Timed tm(c, SPBP_K_INSERT, units, st);
-    return launch_bricks(c, &job, 1, c->bnext, st, t.W0 != nullptr || t.W1 != nullptr);
+    return launch_bricks(c, &job, 1, c->bnext, st, t.W0 != nullptr || t.W1 != nullptr, few);
 }
 
 // PADD2 + batched forward FFT of b images into c->spec.
@@ -1636,10 +1671,9 @@ int spbp_create(const spbp_opts* o, spbp_ctx** out) {
             return bail(fail(nullptr, SPBP_ERR_ALLOC, "twiddle table"));
         c->fft_log2 = L;
     }
-    // default plan: owner-computes bricks, 16x16x13 LDS regions around 12x12x9 cores (the largest region
-    // that runs two 512-thread groups per CU), 128 projections per item: fastest measured at 128^2 into
-    // 256^3 and 256^2 into 512^3; spbp_tune picks per workload
-    if ((rc = configure_bricks(c, NSHAPES - 1))) { std::memcpy(g_last_error, c->err, ERR_LEN); return bail(rc); }
+    // default plan: owner-computes bricks of unit cells (by nearest voxel in launches with few sections), 128
+    // projections per item: fastest measured at 128^2 into 256^3 and 256^2 into 512^3; spbp_tune picks per workload
+    if ((rc = configure_bricks(c, SHAPE_CELLS))) { std::memcpy(g_last_error, c->err, ERR_LEN); return bail(rc); }
     rc = spbp_reset(c, nullptr);
     if (rc) return bail(rc);
     if (hipDeviceSynchronize() != hipSuccess) return bail(fail(nullptr, SPBP_ERR_DEVICE, "zeroing accumulators failed"));
@@ -2000,11 +2034,23 @@ int prepare_batch(const spbp_job* jobs, int njobs) {
     return SPBP_OK;
 }
 
+// Do the brick jobs of round r all hold few sections (one kernel serves them)?
+bool round_few(const spbp_job* jobs, int njobs, int r) {
+    for (int j = 0; j < njobs; ++j) {
+        const spbp_ctx* c = jobs[j].ctx;
+        const int p0 = r * c->fwd_batch;
+        if (p0 >= jobs[j].nimg || own_kernel(c)) continue;
+        if (!few_sections(c, std::min(c->fwd_batch, jobs[j].nimg - p0) * c->nsym)) return false;
+    }
+    return true;
+}
+
 // Host-side job table of round r: the brick jobs of the contexts that still
 // have a chunk in that round (direct- and gather-strategy contexts run their own kernels).
 // Depends only on device addresses, so it can be built before any work runs.
 int round_table(const spbp_job* jobs, int njobs, Geom* const* geom, int r, BrickJob* table, spbp_ctx** lead) {
     int n = 0;
+    const bool few = round_few(jobs, njobs, r);
     *lead = nullptr;
     for (int j = 0; j < njobs; ++j) {
         spbp_ctx* c = jobs[j].ctx;
@@ -2012,7 +2058,7 @@ int round_table(const spbp_job* jobs, int njobs, Geom* const* geom, int r, Brick
         if (p0 >= jobs[j].nimg || own_kernel(c)) continue;
         const Targets t{c->X[0], c->W[0], c->X[1], c->W[1], c->Wc[0], c->Wc[1]};
         const int b = std::min(c->fwd_batch, jobs[j].nimg - p0);
-        table[n++] = brick_job(c, p0, geom[j] + (size_t)p0 * c->nsym, b * c->nsym, t);
+        table[n++] = brick_job(c, p0, geom[j] + (size_t)p0 * c->nsym, b * c->nsym, t, few);
         if (!*lead) *lead = c;   // its list build zeroes its queue head
     }
     return n;
@@ -2030,6 +2076,7 @@ int enqueue_batch(const spbp_job* jobs, int njobs, Geom* const* geom, BrickJob* 
         if (jobs[j].nimg > 0) rounds = std::max(rounds, (jobs[j].nimg + c->fwd_batch - 1) / c->fwd_batch);
     }
     for (int r = 0; r < rounds; ++r) {
+        const bool few = round_few(jobs, njobs, r);
         long units = 0;
         for (int j = 0; j < njobs; ++j) {
             spbp_ctx* c = jobs[j].ctx;
@@ -2045,7 +2092,7 @@ int enqueue_batch(const spbp_job* jobs, int njobs, Geom* const* geom, BrickJob* 
                 if ((rc = launch_own(c, p0, gj, b * c->nsym, t, st, b))) return rc;
                 continue;
             }
-            if ((rc = build_lists(c, gj, b * c->nsym, st))) return rc;
+            if ((rc = build_lists(c, gj, b * c->nsym, st, few))) return rc;
             units += b;
         }
         BrickJob table[MAX_JOBS];
@@ -2053,8 +2100,8 @@ int enqueue_batch(const spbp_job* jobs, int njobs, Geom* const* geom, BrickJob* 
         const int n = round_table(jobs, njobs, geom, r, table, &lead);
         if (!n) continue;
         Timed tm(lead, SPBP_K_INSERT, units, st);
-        const int rc = tables ? launch_bricks_dev(lead, tables[r], n, lead->bnext, st)
-                              : launch_bricks(lead, table, n, lead->bnext, st);
+        const int rc = tables ? launch_bricks_dev(lead, tables[r], n, lead->bnext, st, true, few)
+                              : launch_bricks(lead, table, n, lead->bnext, st, true, few);
         if (rc) return rc;
     }
     return SPBP_OK;
@@ -2812,7 +2859,7 @@ int spbp_scatter_noalloc(int nx, int flags, const float* bi, int nimg, const dou
         int n = 0;
         if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) c.ncu = n;
     }
-    int shape = NSHAPES - 1;
+    int shape = SHAPE_OWN;
     c.bg = grid_of_shape(nx, flags, shape);
     c.shape = shape;
     const int N = c.N, H = c.H;
@@ -2869,10 +2916,10 @@ int spbp_scatter_noalloc(int nx, int flags, const float* bi, int nimg, const dou
         bi_to_raw_kernel<<<nblocks(n), TPB, 0, st>>>((const float2*)bi + (size_t)p0 * N * H, N, H, n, c.spec);
         spec_absmax_kernel<<<b, TPB, 0, st>>>(c.spec, N * H, c.vmax);
         HIPCHK(nullptr, hipGetLastError());
-        if ((rc = build_lists(&c, geom_d, b, st))) return fail(nullptr, rc, "%s", c.err);
-        const BrickJob job = brick_job(&c, 0, geom_d, b, t);
+        if ((rc = build_lists(&c, geom_d, b, st, false))) return fail(nullptr, rc, "%s", c.err);
+        const BrickJob job = brick_job(&c, 0, geom_d, b, t, false);
         HIPCHK(nullptr, hipMemcpyAsync(job_d, &job, sizeof job, hipMemcpyHostToDevice, st));
-        if ((rc = launch_bricks_dev(&c, job_d, 1, c.bnext, st, W != nullptr))) return fail(nullptr, rc, "%s", c.err);
+        if ((rc = launch_bricks_dev(&c, job_d, 1, c.bnext, st, W != nullptr, false))) return fail(nullptr, rc, "%s", c.err);
         // the stack staging (geometry, job table, KB table) is read by the copies above
         HIPCHK(nullptr, hipStreamSynchronize(st));
     }
