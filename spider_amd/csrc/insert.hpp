@@ -1,5 +1,6 @@
 // insert.hpp -- PADD2 and the ONELINE scatter kernels.
 #pragma once
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -139,12 +140,31 @@ __device__ inline void brick_origin(const BrickGrid& bg, int b, int nx, int& x0,
     z0 = -nx + 1 + k * bg.bz;
 }
 
-// The list builders read, per section, only its plane's normal DM(7:9) and its
-// half: packed into 16 bytes (x, y, z, half) so that the (brick, section)
-// tests read a sixth of the section records' bytes.
+// The list builders read, per section, only its plane's normal and its half:
+// packed into 16 bytes (x, y, z, half) so that the (brick, section) tests
+// read a sixth of the section records' bytes.  The normal is the cross
+// product of DM(1:3) and DM(4:6), whose orthonormality the host has checked:
+// a unit vector whatever a caller's DM(7:9) holds, which bounds the bricks a
+// section can hit (plane_hits).
 __global__ __launch_bounds__(TPB) void plane_pack_kernel(const Geom* __restrict__ geom, int n, float4* __restrict__ pln) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < n) pln[p] = make_float4(geom[p].r[6], geom[p].r[7], geom[p].r[8], geom[p].half ? 1.0f : 0.0f);
+    if (p >= n) return;
+    const float* r = geom[p].r;
+    pln[p] = make_float4(r[1] * r[5] - r[2] * r[4], r[2] * r[3] - r[0] * r[5], r[0] * r[4] - r[1] * r[3],
+                         geom[p].half ? 1.0f : 0.0f);
+}
+
+// The most bricks one section's plane can hit: with n its unit normal and a
+// the axis of the largest |n|, the plane crosses a column of bricks along a
+// within |c_a - c*| <= h_a + h_b + h_c + 0.02 / |n_a| of the column's centre
+// line (h: half extents of the bricks' expanded boxes; |n_a| >= 1 / sqrt(3)).
+inline size_t plane_hits(const BrickGrid& bg) {
+    const double mx = bg.own == 1 ? 2.52 : bg.own == 2 ? 0.52 : BRICK_MARGIN, m = bg.own ? 0.52 : BRICK_MARGIN;
+    const double len = 2.0 * (0.5 * (bg.bx - 1) + mx + 0.5 * (bg.by - 1) + m + 0.5 * (bg.bz - 1) + m + 0.1);
+    const size_t cx = (size_t)bg.nby * bg.nbz * std::min(bg.nbx, (int)(len / bg.bx) + 1),
+                 cy = (size_t)bg.nbx * bg.nbz * std::min(bg.nby, (int)(len / bg.by) + 1),
+                 cz = (size_t)bg.nbx * bg.nby * std::min(bg.nbz, (int)(len / bg.bz) + 1);
+    return std::max(cx, std::max(cy, cz));
 }
 
 // A section's plane (through the origin, normal n = DM(7:9)) feeds a brick

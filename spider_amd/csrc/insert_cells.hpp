@@ -93,9 +93,6 @@ struct CellLds {
         y = (((t / TX) % TY) << 2) | ((v >> 2) & 3);
         z = t / (TX * TY);
     }
-    // lattice lines of a section across the cells' box (at most the diagonal + 2), sections a wave takes at a time
-    static constexpr int LINES = (CX + 0.04) * (CX + 0.04) + (CY + 0.04) * (CY + 0.04) + (CZ + 0.04) * (CZ + 0.04) <= 14 * 14 ? 16 : 21;
-    static constexpr int WSEC = 64 / LINES;
     static constexpr int SECS = sizeof(P) == 8 ? CELL_SECS64 : CELL_SECS;
     unsigned long long re[NS], im[NS], w[WGT ? NS : 1];
     float2 val[POOL];                     // the item's samples: value,
@@ -231,37 +228,135 @@ __device__ __forceinline__ int wave_scan(int v) {
     return v;
 }
 
-// A wave's place in the item's sections, kept while it waits for the pool.
+// A wave's place in an item's sections.
 struct CellWalk {
     int s0, q0, total;         // first of the current sections, next point of their sequence, its length
     int start, cnt;            // this lane's line: first point in the sequence, points
     unsigned lrec, open;       // its record; the line open at q0
 };
+// A lattice point of the walk: E = a DM(1:3) + b DM(4:6) of section s, its cell in the brick; `canon`: (a, b) is the
+// sample (I, J) itself, else its Friedel twin (-I, -J).
+template <typename P>
+struct CellPoint {
+    int a, b, s, xc, yc, zc;
+    P x, y, z;
+    bool ok, canon;
+};
+// Lattice lines of a section across the cells' box (at most the diagonal + 2), sections a wave takes at a time.
+template <int CX, int CY, int CZ>
+struct CellLines {
+    static constexpr double D2 = (CX + 0.04) * (CX + 0.04) + (CY + 0.04) * (CY + 0.04) + (CZ + 0.04) * (CZ + 0.04);
+    static constexpr int LINES = D2 <= 14 * 14 ? 16 : 21;
+    static constexpr int WSEC = 64 / LINES;
+    static_assert(D2 <= (LINES - 2) * (LINES - 2), "a section crosses at most the box diagonal + 2 lines");
+};
 
-// Bin the item's sections (geometry buffer `buf`) until they or the pool end;
-// true: the pool ended, call again when it is empty.  A wave takes WSEC
-// sections at a time from L.pnext, LINES lanes each: a lane computes the
-// interval of one lattice line in the cells' box, a scan lays the intervals
-// end to end, and the wave walks them 64 lattice points at a time.  A line's
-// first point among the 64 marks its lane with the line (L.mark); every lane
-// takes the last mark at or before it, or the line that was open before.
-// Two sets of 64 points are in flight: a set's spectrum values are stored
-// while the next set's are on their way.  EDGE: the brick may hold lattice
+// The next sections of the walk (WSEC from *pnext), LINES lanes each: a lane
+// computes the interval of one lattice line in the cells' box, and a scan lays
+// the intervals end to end.  False past the last section (no points then).
+template <int CX, int CY, int CZ, typename P>
+__device__ __forceinline__ bool cell_sections(CellWalk& wk, int* pnext, const P (*g)[6], int ns, int nx, int x0, int y0,
+                                              int z0) {
+    using Ln = CellLines<CX, CY, CZ>;
+    const int lane = threadIdx.x & 63;
+    const int sec = lane / Ln::LINES, line = lane - sec * Ln::LINES;
+    int s0 = 0;
+    if (lane == 0) s0 = atomicAdd(pnext, Ln::WSEC);
+    wk.s0 = __builtin_amdgcn_readfirstlane(s0);
+    wk.q0 = 0;
+    // this lane's line b of section s: lattice points a0 .. a0 + cnt - 1
+    const float lo[3] = {x0 - 0.02f, y0 - 0.02f, z0 - 0.02f};
+    const float hi[3] = {x0 + CX + 0.02f, y0 + CY + 0.02f, z0 + CZ + 0.02f};
+    const int s = min(wk.s0 + sec, ns - 1);
+    float r2[3];
+    float bmn = 0.f, bmx = 0.f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        r2[k] = (float)g[s][3 + k];
+        const float u = r2[k] * lo[k], w = r2[k] * hi[k];
+        bmn += fminf(u, w);
+        bmx += fmaxf(u, w);
+    }
+    const int b = (int)ceilf(bmn - 0.01f) + line;
+    const float bb = (float)b;
+    float amin = -(float)nx, amax = (float)nx;   // |a|, |b| <= nx <= 1024: the records' fields
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        // 1 / DM, |DM| below 10^-6 taken as 10^-6: the line's points then lie inside the box's slab or
+        // outside it for every |a| <= 1024, as they do for the true value
+        const float d = (float)g[s][k], r1 = __builtin_amdgcn_rcpf(fabsf(d) > 1e-6f ? d : 1e-6f);
+        const float off = bb * r2[k];
+        const float u = (lo[k] - off) * r1, w = (hi[k] - off) * r1;
+        amin = fmaxf(amin, fminf(u, w));
+        amax = fminf(amax, fmaxf(u, w));
+    }
+    const int a0 = (int)ceilf(amin - 0.001f);
+    wk.cnt = max(0, (int)floorf(amax + 0.001f) - a0 + 1);
+    if (!(sec < Ln::WSEC && wk.s0 + sec < ns && bb <= bmx + 0.01f && abs(b) <= nx)) wk.cnt = 0;
+    const int pref = wave_scan(wk.cnt);
+    wk.total = __builtin_amdgcn_readlane(pref, 63);
+    wk.start = pref - wk.cnt;
+    // line record: a - q for its points (q: position in the sequence), b, section
+    wk.lrec = (unsigned)(a0 - wk.start + 2048) | ((unsigned)(b + 1024) << 13) | ((unsigned)sec << 25) | 0x80000000u;
+    return wk.s0 < ns;
+}
+
+// The next 64 points of the walk, one per lane (wk.q0 stays).  A line's first
+// point among the 64 marks its lane with the line; every lane takes the last
+// mark at or before it, or the line that was open before.  Returns the
+// record of the line open after the 64.  EDGE: the brick may hold lattice
 // points that are no samples (outside the disk, outside ONELINE's bounds, or
 // the flipped twin at kx = 0).
+template <int CX, int CY, int CZ, bool EDGE, typename P>
+__device__ __forceinline__ unsigned cell_points(CellPoint<P>& t, const CellWalk& wk, unsigned* mark, const P (*g)[6], int ns,
+                                                int nx, int N, int x0, int y0, int z0) {
+    const int lane = threadIdx.x & 63;
+    mark[lane] = 0u;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    if (wk.cnt > 0 && (unsigned)(wk.start - wk.q0) < 64u) mark[wk.start - wk.q0] = wk.lrec;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const unsigned m = mark[lane];
+    const unsigned long long M = __ballot(m != 0u) & ((2ull << lane) - 1ull);
+    unsigned ln = (unsigned)__shfl((int)m, M ? 63 - __clzll((long long)M) : 0, 64);
+    if (!M) ln = wk.open;
+    const int q = wk.q0 + lane;
+    t.a = (int)(ln & 0x1FFFu) - 2048 + q;
+    t.b = (int)((ln >> 13) & 0xFFFu) - 1024;
+    t.s = min(wk.s0 + (int)((ln >> 25) & 3u), ns - 1);
+    cell_pos(g[t.s], t.a, t.b, t.x, t.y, t.z);
+    t.xc = (int)floor(t.x) - x0;
+    t.yc = (int)floor(t.y) - y0;
+    t.zc = (int)floor(t.z) - z0;
+    t.ok = q < wk.total && (unsigned)t.xc < (unsigned)CX && (unsigned)t.yc < (unsigned)CY && (unsigned)t.zc < (unsigned)CZ;
+    t.canon = t.a > 0 || (t.a == 0 && t.b >= 0);
+    if constexpr (EDGE) {
+        t.ok = t.ok && t.a * t.a + t.b * t.b < nx * nx;                   // oneline.f:53-55
+        t.ok = t.ok && (t.canon || t.x > (P)0);                           // oneline.f:60-67 (E_x >= 0 holds)
+        t.ok = t.ok && in_bounds(nearest_voxel(t.x, N), nearest_voxel(t.y, N), nearest_voxel(t.z, N), nx);
+    }
+    return (unsigned)__builtin_amdgcn_readlane((int)ln, 63);
+}
+// May the brick at (x0, y0, z0) hold a lattice point that is no sample?
+template <int CX, int CY, int CZ>
+__device__ __forceinline__ bool cell_edge(int nx, int x0, int y0, int z0) {
+    const int fx = x0 + CX, fy = max(-y0, y0 + CY), fz = max(-z0, z0 + CZ);
+    return x0 == 0 || fx > nx - 3 || y0 < -nx + 4 || y0 + CY > nx - 3 || z0 < -nx + 4 || z0 + CZ > nx - 3 ||
+           fx * fx + fy * fy + fz * fz >= (nx - 1) * (nx - 1);
+}
+
+// Bin the item's sections (geometry buffer `buf`) until they or the pool end;
+// true: the pool ended, call again when it is empty.  Two sets of 64 points
+// are in flight: a set's spectrum values are stored while the next set's are
+// on their way.
 template <int CX, int CY, int CZ, int NT, bool EDGE, bool WGT, typename P>
 __device__ __forceinline__ bool cell_bin(CellLds<CX, CY, CZ, NT, WGT, P>& L, CellWalk& wk, int buf, int ns, int nx, int N,
                                          int x0, int y0, int z0) {
     using Lds = CellLds<CX, CY, CZ, NT, WGT, P>;
-    static_assert((CX + 0.04) * (CX + 0.04) + (CY + 0.04) * (CY + 0.04) + (CZ + 0.04) * (CZ + 0.04) <=
-                      (Lds::LINES - 2) * (Lds::LINES - 2),
-                  "a section crosses at most the box diagonal + 2 lines");
     const int H = nx + 1;
     const int lane = threadIdx.x & 63;
     unsigned* mark = L.mark[threadIdx.x >> 6];
     const P(*g)[6] = L.g[buf];
     const unsigned long long below = (1ull << lane) - 1ull;
-    const int sec = lane / Lds::LINES, line = lane - sec * Lds::LINES;
     // 64 points on their way: record, signs, value, cell, place in the pool (< 0: no sample)
     struct Set {
         unsigned rec, sg;
@@ -272,89 +367,29 @@ __device__ __forceinline__ bool cell_bin(CellLds<CX, CY, CZ, NT, WGT, P>& L, Cel
     // The next 64 points.  No early way out: every set loads, so that the wait for a set's values is for them alone;
     // past the last section or a full pool a set holds no samples.
     auto take = [&](Set& t) {
-        if (wk.q0 >= wk.total) {   // the next sections
-            int s0 = 0;
-            if (lane == 0) s0 = atomicAdd(&L.pnext, Lds::WSEC);
-            wk.s0 = __builtin_amdgcn_readfirstlane(s0);
-            wk.q0 = 0;
-            ended = wk.s0 >= ns;
-            // this lane's line b of section s: lattice points a0 .. a0 + cnt - 1
-            const float lo[3] = {x0 - 0.02f, y0 - 0.02f, z0 - 0.02f};
-            const float hi[3] = {x0 + CX + 0.02f, y0 + CY + 0.02f, z0 + CZ + 0.02f};
-            const int s = min(wk.s0 + sec, ns - 1);
-            float r2[3];
-            float bmn = 0.f, bmx = 0.f;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                r2[k] = (float)g[s][3 + k];
-                const float u = r2[k] * lo[k], w = r2[k] * hi[k];
-                bmn += fminf(u, w);
-                bmx += fmaxf(u, w);
-            }
-            const int b = (int)ceilf(bmn - 0.01f) + line;
-            const float bb = (float)b;
-            float amin = -(float)nx, amax = (float)nx;   // |a|, |b| <= nx <= 1024: the records' fields
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                // 1 / DM, |DM| below 10^-6 taken as 10^-6: the line's points then lie inside the box's slab or
-                // outside it for every |a| <= 1024, as they do for the true value
-                const float d = (float)g[s][k], r1 = __builtin_amdgcn_rcpf(fabsf(d) > 1e-6f ? d : 1e-6f);
-                const float off = bb * r2[k];
-                const float u = (lo[k] - off) * r1, w = (hi[k] - off) * r1;
-                amin = fmaxf(amin, fminf(u, w));
-                amax = fminf(amax, fmaxf(u, w));
-            }
-            const int a0 = (int)ceilf(amin - 0.001f);
-            wk.cnt = max(0, (int)floorf(amax + 0.001f) - a0 + 1);
-            if (!(sec < Lds::WSEC && wk.s0 + sec < ns && bb <= bmx + 0.01f && abs(b) <= nx)) wk.cnt = 0;
-            const int pref = wave_scan(wk.cnt);
-            wk.total = __builtin_amdgcn_readlane(pref, 63);
-            wk.start = pref - wk.cnt;
-            // line record: a - q for its points (q: position in the sequence), b, section
-            wk.lrec = (unsigned)(a0 - wk.start + 2048) | ((unsigned)(b + 1024) << 13) | ((unsigned)sec << 25) | 0x80000000u;
-        }
-        mark[lane] = 0u;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        if (wk.cnt > 0 && (unsigned)(wk.start - wk.q0) < 64u) mark[wk.start - wk.q0] = wk.lrec;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        const unsigned m = mark[lane];
-        const unsigned long long M = __ballot(m != 0u) & (below | (1ull << lane));
-        unsigned ln = (unsigned)__shfl((int)m, M ? 63 - __clzll((long long)M) : 0, 64);
-        if (!M) ln = wk.open;
-        const int q = wk.q0 + lane;
-        const int a = (int)(ln & 0x1FFFu) - 2048 + q, b = (int)((ln >> 13) & 0xFFFu) - 1024;
-        const int s = min(wk.s0 + (int)((ln >> 25) & 3u), ns - 1);
-        P x, y, z;
-        cell_pos(g[s], a, b, x, y, z);
-        const int xc = (int)floor(x) - x0, yc = (int)floor(y) - y0, zc = (int)floor(z) - z0;
-        bool ok = q < wk.total && (unsigned)xc < (unsigned)CX && (unsigned)yc < (unsigned)CY && (unsigned)zc < (unsigned)CZ;
-        const bool canon = a > 0 || (a == 0 && b >= 0);   // the sample (I, J) itself, not its twin (-I, -J)
-        if constexpr (EDGE) {
-            ok = ok && a * a + b * b < nx * nx;                       // oneline.f:53-55
-            ok = ok && (canon || x > (P)0);                           // oneline.f:60-67 (E_x >= 0 holds)
-            ok = ok && in_bounds(nearest_voxel(x, N), nearest_voxel(y, N), nearest_voxel(z, N), nx);
-        }
-        const unsigned long long mk = __ballot(ok);
+        if (wk.q0 >= wk.total) ended = !cell_sections<CX, CY, CZ, P>(wk, &L.pnext, g, ns, nx, x0, y0, z0);
+        CellPoint<P> p;
+        const unsigned open = cell_points<CX, CY, CZ, EDGE, P>(p, wk, mark, g, ns, nx, N, x0, y0, z0);
+        const unsigned long long mk = __ballot(p.ok);
         const int n = (int)__popcll(mk);
         int base = 0;
         if (lane == 0) base = atomicAdd(&L.npool, n);
         {
             // spectrum_value: sign (-1)^(I + J), conjugated, and conjugated back for a flipped sample.  Every lane
-            // loads, the section's first value
-            // where no sample is
-            const int I = canon ? a : -a, J = canon ? b : -b;
-            t.val = *(Global<const f2v>)(as_global(L.spec[buf][s]) + (ok ? (J >= 0 ? J : J + N) * H + I : 0));
+            // loads, the section's first value where no sample is
+            const int I = p.canon ? p.a : -p.a, J = p.canon ? p.b : -p.b;
+            t.val = *(Global<const f2v>)(as_global(L.spec[buf][p.s]) + (p.ok ? (J >= 0 ? J : J + N) * H + I : 0));
         }
-        t.sg = ((unsigned)((a + b) & 1) << 31) | (canon ? 1u : 0u);
-        t.rec = cell_rec(a, b, s);
-        t.cell = (zc * CY + yc) * CX + xc;
+        t.sg = ((unsigned)((p.a + p.b) & 1) << 31) | (p.canon ? 1u : 0u);
+        t.rec = cell_rec(p.a, p.b, p.s);
+        t.cell = (p.zc * CY + p.yc) * CX + p.xc;
         base = __builtin_amdgcn_readfirstlane(base);
         // no room: these points again when the pool is empty (npool stays past its end until then)
         const bool room = base + n <= Lds::POOL;
-        t.slot = ok && room ? base + (int)__popcll(mk & below) : -1;
+        t.slot = p.ok && room ? base + (int)__popcll(mk & below) : -1;
         blocked = !room;
         if (room) {
-            wk.open = (unsigned)__builtin_amdgcn_readlane((int)ln, 63);
+            wk.open = open;
             wk.q0 += 64;
         }
     };
@@ -459,10 +494,7 @@ __device__ __forceinline__ void cell_load(CellLds<CX, CY, CZ, NT, WGT, P>& L, in
         brick_origin(J.bg, b, nx, c.x0, c.y0, c.z0);
         c.half = half;
         c.ns = ns;
-        // can the brick hold a lattice point that is no sample?
-        const int fx = c.x0 + CX, fy = max(-c.y0, c.y0 + CY), fz = max(-c.z0, c.z0 + CZ);
-        c.edge = c.x0 == 0 || fx > nx - 3 || c.y0 < -nx + 4 || c.y0 + CY > nx - 3 || c.z0 < -nx + 4 || c.z0 + CZ > nx - 3 ||
-                 fx * fx + fy * fy + fz * fz >= (nx - 1) * (nx - 1);
+        c.edge = cell_edge<CX, CY, CZ>(nx, c.x0, c.y0, c.z0);
         // fixed-point unit (as insert_brick_kernel's): terms below 2^VBITS units
         c.e = 0;
         if (m > 0.0f && isfinite(m)) (void)frexpf(m, &c.e);

@@ -50,6 +50,7 @@
 #include "insert_cells.hpp"
 #include "insert_gather.hpp"
 #include "project.hpp"
+#include "project_cells.hpp"
 #include "resolve.hpp"
 #include "rotate.hpp"
 
@@ -384,7 +385,8 @@ int ensure_lists(spbp_ctx* c, int B) {
         const int rc = configure_bricks(c, c->shape);
         if (rc) return rc;
     }
-    const size_t cap = (size_t)B * c->nsym * c->bg.nb;   // B images, nsym sections each
+    // B images, nsym sections each, and the bricks a section hits at most (of either grid of the unit-cell shape)
+    const size_t cap = (size_t)B * c->nsym * std::max(plane_hits(c->bg), c->bgo.nb > 0 ? plane_hits(c->bgo) : 0);
     const size_t ns = (size_t)B * c->nsym;
     if (c->blist && c->bikey && c->blist_cap >= cap && c->bpln && c->bpln_cap >= ns) return SPBP_OK;
     if (c->graphs > 0) return refuse_captured(c, "growing the brick lists");
@@ -712,7 +714,7 @@ int launch_bricks(spbp_ctx* c, const BrickJob* jh, int n, int* counter, hipStrea
 // also zeroes c's queue head.
 int build_lists(spbp_ctx* c, const Geom* geom_d, int b, hipStream_t st, bool few) {
     const BrickGrid& bg = few ? c->bgo : c->bg;
-    if (c->bg.nb <= 0 || bg.nb > c->bg.nb || !c->bcnt || !c->blist || !c->bikey || c->blist_cap < (size_t)b * c->bg.nb || !c->bpln ||
+    if (c->bg.nb <= 0 || bg.nb > c->bg.nb || !c->bcnt || !c->blist || !c->bikey || c->blist_cap < (size_t)b * plane_hits(bg) || !c->bpln ||
         c->bpln_cap < (size_t)b)
         return fail(c, SPBP_ERR_ARG, "brick lists not allocated for %d sections", b);
     const int nkeys = 2 * bg.nb;
@@ -860,6 +862,54 @@ int pad_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
         FFTCHK(c, hipfftExecR2C(plan, (hipfftReal*)c->padbuf, (hipfftComplex*)c->spec));
     }
     spec_absmax_kernel<<<b, TPB, 0, st>>>(c->spec, c->N * c->H, c->vmax);
+    HIPCHK(c, hipGetLastError());
+    return SPBP_OK;
+}
+
+// Central-slice gather of b sections (geometry at geom_d, image numbers from
+// img0) of the half grid X into out (b spectra in the BI layout): by bricks
+// of unit cells where the context has their lists (the default shape) and the
+// launch enough samples, else sample by sample from memory.  A live batch
+// graph replays work on the lists, maybe on another stream: then, too, the
+// second.  The lists, the zero fill and the bricks' regions cost ~60 us and
+// more for larger grids: from NX sections and 2^19 pixels they are repaid
+// (by samples / by bricks, us: 64^2, 128 sections 103 / 102, 256 175 / 121;
+// 128^2, 128 314 / 247, 2048 4461 / 1425; 32^2, 100 38 / 65, 800 138 / 119;
+// 256^2, 256 2472 / 1519).
+bool gather_by_bricks(const spbp_ctx* c, int b) {
+    return c->shape == SHAPE_CELLS && c->graphs == 0 && b >= c->nx && (size_t)b * c->nx * c->nx >= (size_t)1 << 19;
+}
+
+int launch_slices(spbp_ctx* c, const float2* X, const Geom* geom_d, int img0, int b, float2* out, hipStream_t st) {
+    const int N = c->N, H = c->H;
+    const bool f64 = (c->flags & SPBP_GEOM_F64) != 0;
+    Timed tm(c, SPBP_K_GATHER, b, st);
+    if (gather_by_bricks(c, b) && c->blist && c->bikey && c->bpln_cap >= (size_t)b &&
+        c->blist_cap >= (size_t)b * plane_hits(c->bg)) {
+        fill((float*)out, 2 * (size_t)b * N * H, 0.0f, st);   // only samples are written
+        int rc = build_lists(c, geom_d, b, st, false);
+        if (rc) return rc;
+        const unsigned grid = (unsigned)c->ncu * GATHER_GROUPS;
+        static_assert(GATHER_SECS >= CELL_SECS && GATHER_SECS >= CELL_SECS64, "the lists' items fit the gather's");
+        if (f64)
+            gather_cells_kernel<double><<<grid, GATHER_NT, 0, st>>>(X, geom_d, img0, c->bg, c->nx, N, c->tab, c->fltb, c->bcnt,
+                                                                    c->boff, c->bioff, c->bikey, c->blist, out, c->bnext);
+        else
+            gather_cells_kernel<float><<<grid, GATHER_NT, 0, st>>>(X, geom_d, img0, c->bg, c->nx, N, c->tab, c->fltb, c->bcnt,
+                                                                   c->boff, c->bioff, c->bikey, c->blist, out, c->bnext);
+        HIPCHK(c, hipGetLastError());
+        return SPBP_OK;
+    }
+    const unsigned gx = (unsigned)(((H + GT - 1) / GT) * ((N + GT - 1) / GT));
+    for (int q0 = 0; q0 < b; q0 += 65535) {
+        const int bq = std::min(65535, b - q0);
+        if (f64)
+            gather_kernel<double><<<dim3(gx, bq), GT * GT, 0, st>>>(X, geom_d + q0, c->nx, N, c->tab, c->fltb,
+                                                                    out + (size_t)q0 * N * H);
+        else
+            gather_kernel<float><<<dim3(gx, bq), GT * GT, 0, st>>>(X, geom_d + q0, c->nx, N, c->tab, c->fltb,
+                                                                   out + (size_t)q0 * N * H);
+    }
     HIPCHK(c, hipGetLastError());
     return SPBP_OK;
 }
@@ -1766,19 +1816,14 @@ int spbp_gather(spbp_ctx* c, const float* X, int nimg, const double* angles_deg,
     hipStream_t st = (hipStream_t)stream;
     int rc = stage_geom(c, nimg, dm, angles_deg, nullptr, st, false);
     if (rc) return rc;
-    const int N = c->N, H = c->H;
-    const unsigned gx = (unsigned)(((H + GT - 1) / GT) * ((N + GT - 1) / GT));
-    for (int p0 = 0; p0 < nimg; p0 += 65535) {
-        const int b = std::min(65535, nimg - p0);
-        Timed tm(c, SPBP_K_GATHER, b, st);
-        if (c->flags & SPBP_GEOM_F64)
-            gather_kernel<double><<<dim3(gx, b), GT * GT, 0, st>>>((const float2*)X, c->geom_d + p0, c->nx, N, c->tab,
-                                                                   c->fltb, (float2*)out_bi + (size_t)p0 * N * H);
-        else
-            gather_kernel<float><<<dim3(gx, b), GT * GT, 0, st>>>((const float2*)X, c->geom_d + p0, c->nx, N, c->tab,
-                                                                  c->fltb, (float2*)out_bi + (size_t)p0 * N * H);
+    // the brick lists, where they can be had: without them the gather reads the grid sample by sample
+    const int B = std::min(c->batch, nimg);
+    if (gather_by_bricks(c, B) && ensure_lists(c, B) != SPBP_OK) (void)hipGetLastError();
+    for (int p0 = 0; p0 < nimg; p0 += B) {
+        const int b = std::min(B, nimg - p0);
+        if ((rc = launch_slices(c, (const float2*)X, c->geom_d + p0, p0, b, (float2*)out_bi + (size_t)p0 * c->N * c->H, st)))
+            return rc;
     }
-    HIPCHK(c, hipGetLastError());
     return SPBP_OK;
 }
 
@@ -1826,7 +1871,6 @@ int spbp_gather_images(spbp_ctx* c, const float* X, int nimg, const double* angl
         c->c2r_cap = B;
     }
     const int ip = (N - c->nx) / 2 + c->nx % 2;
-    const unsigned gx = (unsigned)(((H + GT - 1) / GT) * ((N + GT - 1) / GT));
     for (int p0 = 0; p0 < nimg; p0 += B) {
         const int b = std::min(B, nimg - p0);
         // a plan per batch size, two kept: the most recent becomes c2r
@@ -1843,18 +1887,7 @@ int spbp_gather_images(spbp_ctx* c, const float* X, int nimg, const double* angl
             if (r != HIPFFT_SUCCESS) { c->c2r = 0; return fail(c, SPBP_ERR_FFT, "hipfftPlanMany(C2R %d): %d", b, (int)r); }
             c->c2r_batch = b;
         }
-        {
-            Timed tm(c, SPBP_K_GATHER, b, st);
-            for (int q0 = 0; q0 < b; q0 += 65535) {
-                const int bq = std::min(65535, b - q0);
-                if (c->flags & SPBP_GEOM_F64)
-                    gather_kernel<double><<<dim3(gx, bq), GT * GT, 0, st>>>((const float2*)X, c->geom_d + p0 + q0, c->nx,
-                                                                            N, c->tab, c->fltb, c->spec + (size_t)q0 * N * H);
-                else
-                    gather_kernel<float><<<dim3(gx, bq), GT * GT, 0, st>>>((const float2*)X, c->geom_d + p0 + q0, c->nx,
-                                                                           N, c->tab, c->fltb, c->spec + (size_t)q0 * N * H);
-            }
-        }
+        if ((rc = launch_slices(c, (const float2*)X, c->geom_d + p0, p0, b, c->spec, st))) return rc;
         const size_t n = (size_t)b * N * H;
         bi_complete_kernel<<<nblocks(n), TPB, 0, st>>>(c->spec, N, H, c->nx, n);
         HIPCHK(c, hipGetLastError());
