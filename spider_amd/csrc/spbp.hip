@@ -44,6 +44,7 @@
 #include "calib.hpp"
 #include "common.hpp"
 #include "fft.hpp"
+#include "fft_any.hpp"
 #include "finalize.hpp"
 #include "hostmath.hpp"
 #include "insert.hpp"
@@ -137,7 +138,9 @@ struct spbp_ctx {
     int c2r_cap = 0;
     // own forward transforms (power-of-two N): e^{-2 pi i m / N}, m < N
     float2* tw = nullptr;
-    int fft_log2 = 0;   // log2 N, or 0 when hipFFT does the forward transforms
+    int fft_log2 = 0;   // log2 N of a power of two the own transforms take, else 0
+    FftPlan fft{};      // the own transforms' passes for other N = 2^a 3^b 5^c 7^d (np > 0)
+    bool own_fwd() const { return fft_log2 > 0 || fft.np > 0; }   // else hipFFT does the forward transforms
     double* fmean = nullptr;   // per chunk image: PADD2's mean
     // finalisation
     hipfftHandle inv = 0;
@@ -408,24 +411,25 @@ int ensure_lists(spbp_ctx* c, int B) {
 // want_batch projections.  c->fwd_batch is the committed chunk size: zero
 // until every buffer of the set exists.
 int ensure_chunk(spbp_ctx* c, int want_batch) {
-    const bool set = c->spec && c->vmax && (c->fft_log2 ? c->fmean != nullptr : (c->padbuf && c->fwd));
+    const bool set = c->spec && c->vmax && (c->own_fwd() ? c->fmean != nullptr : (c->padbuf && c->fwd));
     if (set && c->fwd_batch >= want_batch) return ensure_lists(c, c->fwd_batch);
     if (c->graphs > 0) return refuse_captured(c, "growing the chunk buffers");
     c->fwd_batch = 0;
     if (c->padbuf) { (void)hipFree(c->padbuf); c->padbuf = nullptr; }
     if (c->spec) { (void)hipFree(c->spec); c->spec = nullptr; }
     if (c->fwd) { hipfftDestroy(c->fwd); c->fwd = 0; }
-    if (c->fwd_tail) { hipfftDestroy(c->fwd_tail); c->fwd_tail = 0; c->tail_batch = 0; }
+    if (c->fwd_tail) { hipfftDestroy(c->fwd_tail); c->fwd_tail = 0; }
+    c->tail_batch = 0;
     if (c->vmax) { (void)hipFree(c->vmax); c->vmax = nullptr; }
     if (c->fmean) { (void)hipFree(c->fmean); c->fmean = nullptr; }
     const int N = c->N, H = c->H, B = want_batch;
-    if (!c->fft_log2) HIPCHK(c, dmalloc(&c->padbuf, (size_t)B * N * N * sizeof(float)));
+    if (!c->own_fwd()) HIPCHK(c, dmalloc(&c->padbuf, (size_t)B * N * N * sizeof(float)));
     HIPCHK(c, dmalloc(&c->spec, (size_t)B * N * H * sizeof(float2)));
     HIPCHK(c, dmalloc(&c->vmax, (size_t)B * sizeof(float)));
-    if (c->fft_log2) HIPCHK(c, dmalloc(&c->fmean, (size_t)B * sizeof(double)));
+    if (c->own_fwd()) HIPCHK(c, dmalloc(&c->fmean, (size_t)B * sizeof(double)));
     int rc = ensure_lists(c, B);
     if (rc) return rc;
-    if (!c->fft_log2) {   // own transforms need no plan, and the pad buffer is not used
+    if (!c->own_fwd()) {   // own transforms need no plan, and the pad buffer is not used
         int n[2] = {N, N};
         int inembed[2] = {N, N};
         int onembed[2] = {N, H};
@@ -433,6 +437,17 @@ int ensure_chunk(spbp_ctx* c, int want_batch) {
         if (r != HIPFFT_SUCCESS) { c->fwd = 0; return fail(c, SPBP_ERR_FFT, "hipfftPlanMany(%d): hipfft error %d", B, (int)r); }
     }
     c->fwd_batch = B;
+    return SPBP_OK;
+}
+
+// A partial chunk under a live batch graph: only the chunk size and the last
+// partial size set before are taken, whoever does the transforms.  (hipFFT
+// needs a plan per size; callers see one rule for every N that is no power of
+// two.)
+int tail_ok(spbp_ctx* c, int b) {
+    if (b == c->fwd_batch || b == c->tail_batch) return SPBP_OK;
+    if (c->graphs > 0) return refuse_captured(c, "a new forward FFT plan");
+    c->tail_batch = b;
     return SPBP_OK;
 }
 
@@ -795,12 +810,11 @@ int run_insert(spbp_ctx* c, int img0, const Geom* geom_d, int ng, const Targets&
 }
 
 // PADD2 + batched forward FFT of b images into c->spec.
-// The own two-pass R2C of b zero-padded images minus c->fmean[i] into c->spec
-// (power-of-two N); c->vmax receives each spectrum's largest |Re|, |Im| and
+// The own two-pass R2C of b zero-padded images minus c->fmean[i] into c->spec; c->vmax receives each spectrum's largest |Re|, |Im| and
 // must be zero on entry.
 int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
     const size_t lds = fft_lds_bytes(c->N), rlds = fft_lds_bytes(c->N, FFT_ROW_ELEMS);
-    const int M = std::min(FFT_ROW_ELEMS / c->N, c->nx / 2);   // >= 1: own transforms need N <= FFT_ROW_ELEMS
+    const int pairs = (c->nx + 1) / 2, M = std::min(FFT_ROW_ELEMS / c->N, pairs);   // >= 1: own transforms need N <= FFT_ROW_ELEMS
     const int cw = FFT_ELEMS / c->N;
     const size_t npix = (size_t)c->nx * c->nx, nspec = (size_t)c->N * c->H;
     const size_t esz = dtype == SPBP_BF16 ? 2 : 4;
@@ -816,8 +830,12 @@ int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
         float2* sp = c->spec + s0 * nspec;
         {
             Timed tm(c, SPBP_K_PAD, n, st);
-            const dim3 rgrid((c->nx / 2 + M - 1) / M, n);
-            if (dtype == SPBP_BF16)
+            const dim3 rgrid((pairs + M - 1) / M, n);
+            if (!c->fft_log2 && dtype == SPBP_BF16)
+                row_any_kernel<uint16_t><<<rgrid, TPB, rlds, st>>>((const uint16_t*)im, c->nx, c->fft, c->tw, c->fmean + s0, sp);
+            else if (!c->fft_log2)
+                row_any_kernel<float><<<rgrid, TPB, rlds, st>>>((const float*)im, c->nx, c->fft, c->tw, c->fmean + s0, sp);
+            else if (dtype == SPBP_BF16)
                 row_fft_kernel<uint16_t><<<rgrid, TPB, rlds, st>>>((const uint16_t*)im, c->nx, c->N, c->fft_log2, c->tw,
                                                                   c->fmean + s0, sp);
             else
@@ -826,8 +844,11 @@ int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
         }
         {
             Timed tm(c, SPBP_K_FFT2, n, st);
-            col_fft_kernel<<<dim3((c->H + cw - 1) / cw, n), FFT_COL_NT, lds, st>>>(c->nx, c->N, c->fft_log2, c->tw, sp,
-                                                                           c->vmax + s0);
+            const dim3 cgrid((c->H + cw - 1) / cw, n);
+            if (c->fft_log2)
+                col_fft_kernel<<<cgrid, FFT_COL_NT, lds, st>>>(c->nx, c->N, c->fft_log2, c->tw, sp, c->vmax + s0);
+            else
+                col_any_kernel<<<cgrid, FFT_COL_NT, lds, st>>>(c->nx, c->fft, c->tw, sp, c->vmax + s0);
         }
     }
     HIPCHK(c, hipGetLastError());
@@ -835,10 +856,18 @@ int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
 }
 
 int pad_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
-    if (c->fft_log2) {
+    if (c->own_fwd()) {
+        if (!c->fft_log2) {
+            int rc = tail_ok(c, b);
+            if (rc) return rc;
+        }
         {
             Timed tm(c, SPBP_K_PAD, b, st);   // the means of the whole chunk (one block per image)
-            if (dtype == SPBP_BF16)
+            if (!c->fft_log2 && dtype == SPBP_BF16)
+                pad_mean_any_kernel<uint16_t><<<b, TPB, 0, st>>>((const uint16_t*)src, c->nx, c->fmean, c->vmax);
+            else if (!c->fft_log2)
+                pad_mean_any_kernel<float><<<b, TPB, 0, st>>>((const float*)src, c->nx, c->fmean, c->vmax);
+            else if (dtype == SPBP_BF16)
                 pad_mean_kernel<uint16_t><<<b, TPB, 0, st>>>((const uint16_t*)src, c->nx, c->fft_log2 - 1, c->fmean, c->vmax);
             else
                 pad_mean_kernel<float><<<b, TPB, 0, st>>>((const float*)src, c->nx, c->fft_log2 - 1, c->fmean, c->vmax);
@@ -1708,9 +1737,8 @@ int spbp_create(const spbp_opts* o, spbp_ctx** out) {
         hipEventCreateWithFlags(&c->jobs_evt, hipEventDisableTiming) != hipSuccess)
         return bail(fail(nullptr, SPBP_ERR_DEVICE, "context set-up failed"));
     if (dmalloc(&c->bnext, sizeof(int)) != hipSuccess) return bail(fail(nullptr, SPBP_ERR_ALLOC, "brick queue"));
-    if ((c->N & (c->N - 1)) == 0 && c->N >= 8 && c->N <= std::min(2048, FFT_ROW_ELEMS) && !(o->flags & SPBP_HIPFFT)) {
-        int L = 0;
-        while ((1 << L) < c->N) ++L;
+    const FftPlan fp = fft_plan(c->N);
+    if (fp.np && !(o->flags & SPBP_HIPFFT)) {
         std::vector<float2> t(c->N);
         for (int m = 0; m < c->N; ++m) {
             const double a = -2.0 * M_PI * (double)m / (double)c->N;
@@ -1719,7 +1747,10 @@ int spbp_create(const spbp_opts* o, spbp_ctx** out) {
         if (dmalloc(&c->tw, t.size() * sizeof(float2)) != hipSuccess ||
             hipMemcpy(c->tw, t.data(), t.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess)
             return bail(fail(nullptr, SPBP_ERR_ALLOC, "twiddle table"));
-        c->fft_log2 = L;
+        if ((c->N & (c->N - 1)) == 0)
+            while ((1 << c->fft_log2) < c->N) ++c->fft_log2;
+        else
+            c->fft = fp;
     }
     // default plan: owner-computes bricks of unit cells (by nearest voxel in launches with few sections), 128
     // projections per item: fastest measured at 128^2 into 256^3 and 256^2 into 512^3; spbp_tune picks per workload
