@@ -48,6 +48,19 @@ __device__ inline void block_sum2(double& s, unsigned& c) {
     }
 }
 
+// A pointer read from a job record is generic to the compiler, whose FLAT
+// accesses count as LDS accesses too: a wait for one drains the wave's LDS
+// atomics.  These types and accessors make them global accesses.
+#define SPBP_AS1 __attribute__((address_space(1)))
+template <typename T> using Global = SPBP_AS1 T*;
+template <typename T>
+__device__ __forceinline__ Global<T> as_global(T* p) { return (Global<T>)p; }
+typedef float f2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float2 load2(Global<const float2> p) {
+    const f2v v = *(Global<const f2v>)p;
+    return make_float2(v.x, v.y);
+}
+__device__ __forceinline__ void store2(Global<float2> p, float2 v) { *(Global<f2v>)p = f2v{v.x, v.y}; }
 
 // p[0 .. n) = v, four values per thread (one 16-byte store when p is
 // 16-byte aligned).  Launched by fill(): a kernel, not hipMemsetAsync, so that

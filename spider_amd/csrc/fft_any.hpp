@@ -19,17 +19,18 @@ struct FftPlan {
     int N, np;
     int R[ANY_PASSES], Ns[ANY_PASSES];
     unsigned mq[ANY_PASSES], mNs[ANY_PASSES];   // by N / R and by Ns
-    unsigned mN, mH;                            // by N and by N / 2 + 1
+    unsigned mN, mH, mL;                        // by N, by N / 2 + 1 and by N / 2
 };
 inline unsigned recip(int d) { return (unsigned)((1ull << 32) / (unsigned)d + 1); }   // d >= 2
 
 // The plan of N, or np = 0 when N is no product of 2, 3, 5 and 7 (or too large for a block).
 inline FftPlan fft_plan(int N) {
     FftPlan p{};
+    if (N < 8 || N > FFT_ROW_ELEMS) return p;
     p.N = N;
     p.mN = recip(N);
     p.mH = recip(N / 2 + 1);
-    if (N < 8 || N > FFT_ROW_ELEMS) return p;
+    p.mL = recip(N / 2);
     int n = N, np = 0, Ns = 1;
     const int rad[5] = {7, 5, 3, 4, 2};
     for (int r : rad)

@@ -1,6 +1,7 @@
 // finalize.hpp -- SYMPLANE0 / NRMW2 / WINDKB2A kernels and partial volumes.
 #pragma once
 #include "common.hpp"
+#include "fft_any.hpp"
 
 namespace spbp {
 
@@ -49,16 +50,11 @@ __device__ inline void load_sym(const Acc& a, int nx, int N, int i, int j, int k
     }
 }
 
-__device__ inline float2 norm_val(const Acc& a, int nx, int N, int i, int j, int k) {
-    float2 x;
-    float w;
-    double wd;
-    load_sym(a, nx, N, i, j, k, x, w, wd);
-    const float s = ((i + j + k) & 1) ? -1.0f : 1.0f;
-    // NRMW2 (bp3f.f:1359): divide where W > 0.1; near 0.1 the decision may
-    // come from the reference's own sums
-    const unsigned char m = a.mask ? (a.mask[((size_t)k * N + j) * (nx + 1) + i] >> a.mshift) & 3 : 0;
-    if (a.Wc[0]) {
+// NRMW2 (bp3f.f:1359) of one voxel: divide where W > 0.1; near 0.1 the decision
+// m may come from the reference's own sums.  odd: parity of i + j + k.
+__device__ inline float2 norm_div(bool comp, float2 x, float w, double wd, int m, int odd) {
+    const float s = odd ? -1.0f : 1.0f;
+    if (comp) {
         // compensated weights: threshold and division in FP64
         if (m ? m == 2 : wd > (double)0.1f)
             return make_float2((float)((double)(x.x * s) / wd), (float)((double)(x.y * s) / wd));
@@ -69,35 +65,62 @@ __device__ inline float2 norm_val(const Acc& a, int nx, int N, int i, int j, int
     return make_float2(0.f, 0.f);
 }
 
+__device__ inline float2 norm_val(const Acc& a, int nx, int N, int i, int j, int k) {
+    float2 x;
+    float w;
+    double wd;
+    load_sym(a, nx, N, i, j, k, x, w, wd);
+    const int m = a.mask ? (a.mask[((size_t)k * N + j) * (nx + 1) + i] >> a.mshift) & 3 : 0;
+    return norm_div(a.Wc[0] != nullptr, x, w, wd, m, (i + j + k) & 1);
+}
+
 // ------------------------------------------------------------------ batched finalisation
+// The own inverse transform's blocks (inverse.hpp): 16 columns of N = 256 (8 of
+// 512).
+constexpr int INV_ELEMS = 4096, INV_NT = 512;
+constexpr int INV_LDS = INV_ELEMS + 96;   // columns are N + 1 apart; min(N / 2 + 1, INV_ELEMS / N) <= 65 of them
+inline int inv_slabs(int N) { const int cw = INV_ELEMS / N; return (N / 2 + 1 + cw - 1) / cw; }
+// Row pairs per block of the x pass: up to FFT_ROW_ELEMS values, but 256 blocks where the volume has them.
+inline int inv_pairs(int nx) {
+    const int all = (nx * nx + 1) / 2;
+    return std::max(1, std::min(FFT_ROW_ELEMS / (2 * nx), all / 256));
+}
+inline unsigned inv_x_blocks(int nx) { return (unsigned)(((nx * nx + 1) / 2 + inv_pairs(nx) - 1) / inv_pairs(nx)); }
+
 // One volume of a batched finalisation: its accumulators, transform buffers,
-// output and its first block in each of the two grids one launch covers (the
-// half-grid grid of the normalisation, the NX^3 grid of the window steps).
-// A launch covers a contiguous run of jobs; block offsets are relative to the
+// output and its first block in each of the grids the launches cover.  A
+// launch covers a contiguous run of jobs; block offsets are relative to the
 // run's first job.
 struct FinalJob {
     Acc a;
-    float2* work;          // half-complex input of the inverse transform
-    const float* real;     // its N^3 output
+    float2* work;          // half-complex input of the inverse transform, or the own passes' intermediates
+    const float* real;     // hipFFT's N^3 output
     float* out;            // NX^3 volume
     const float* wkb;      // WINDKB2A divisor by squared radius
-    double* psum;          // per volume block: outer-shell sum and count
+    double* psum;          // per window block: outer-shell sum and count
     unsigned* pcnt;
     float* mean;
     int nx, N;
     float pix;             // 1 / N^3
-    unsigned hb0, vb0;     // first block in the half-grid / volume grid
-    unsigned vnb;          // volume blocks
+    unsigned hb0, vb0;     // first block in the half-grid (y pass) / volume grid
+    unsigned vnb;          // window blocks
     double invH, invN, invL;   // 1 / (NX + 1), 1 / N, 1 / NX
+    // own inverse transform
+    unsigned zb0, xb0;     // first block in the grids of the z and x passes
+    int slabs, pairs;      // column slabs per plane; row pairs per block of the x pass
+    const float2* tw;
+    FftPlan fft;
 };
 
-// Job of block b: the last of the run whose first block is <= b.
-template <bool VOL>
+// Job of block b: the last of the run whose first block is <= b.  Grids: 0 half
+// grid (y pass), 1 z pass, 2 x pass, 3 volume.
+template <int GRID>
 __device__ inline int job_of_block(const FinalJob* __restrict__ jobs, int nj, unsigned b) {
     int lo = 0, hi = nj - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if ((VOL ? jobs[mid].vb0 : jobs[mid].hb0) <= b) lo = mid;
+        const FinalJob& f = jobs[mid];
+        if ((GRID == 0 ? f.hb0 : GRID == 1 ? f.zb0 : GRID == 2 ? f.xb0 : f.vb0) <= b) lo = mid;
         else hi = mid - 1;
     }
     return lo;
@@ -109,7 +132,7 @@ __device__ inline int job_of_block(const FinalJob* __restrict__ jobs, int nj, un
 constexpr int NORM_VPT = 4;
 
 __global__ __launch_bounds__(TPB) void normalize_kernel(const FinalJob* __restrict__ jobs, int nj) {
-    const FinalJob& f = jobs[job_of_block<false>(jobs, nj, blockIdx.x)];
+    const FinalJob& f = jobs[job_of_block<0>(jobs, nj, blockIdx.x)];
     const int nx = f.nx, N = f.N, H = nx + 1;
     const size_t total = (size_t)H * N * N;
     const size_t base = (size_t)(blockIdx.x - f.hb0) * (TPB * NORM_VPT) + threadIdx.x;
@@ -136,7 +159,7 @@ __global__ __launch_bounds__(TPB) void normalize_kernel(const FinalJob* __restri
 
 // ------------------------------------------------------------------ WINDKB2A
 __global__ __launch_bounds__(TPB) void window_kernel(const FinalJob* __restrict__ jobs, int nj) {
-    const FinalJob& f = jobs[job_of_block<true>(jobs, nj, blockIdx.x)];
+    const FinalJob& f = jobs[job_of_block<3>(jobs, nj, blockIdx.x)];
     const int L = f.nx, N = f.N;
     const unsigned lb = blockIdx.x - f.vb0;
     const size_t total = (size_t)L * L * L;
@@ -173,7 +196,7 @@ __global__ __launch_bounds__(TPB) void shell_mean_kernel(const FinalJob* __restr
 }
 
 __global__ __launch_bounds__(TPB) void subtract_kernel(const FinalJob* __restrict__ jobs, int nj) {
-    const FinalJob& f = jobs[job_of_block<true>(jobs, nj, blockIdx.x)];
+    const FinalJob& f = jobs[job_of_block<3>(jobs, nj, blockIdx.x)];
     const int L = f.nx;
     const size_t total = (size_t)L * L * L;
     const size_t idx = (size_t)(blockIdx.x - f.vb0) * blockDim.x + threadIdx.x;

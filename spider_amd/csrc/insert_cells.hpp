@@ -54,18 +54,6 @@ constexpr int CELL_WBITS = 48;
 constexpr double CELL_WSCALE = 281474976710656.0;          // 2^48
 constexpr double CELL_WINV = 1.0 / 281474976710656.0;
 
-// A pointer read from a job record is generic to the compiler, whose FLAT
-// accesses count as LDS accesses too: a wait for one drains the wave's LDS
-// atomics.  These types and accessors make them global accesses.
-#define SPBP_AS1 __attribute__((address_space(1)))
-template <typename T> using Global = SPBP_AS1 T*;
-template <typename T>
-__device__ __forceinline__ Global<T> as_global(T* p) { return (Global<T>)p; }
-typedef float f2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float2 load2(Global<const float2> p) {
-    const f2v v = *(Global<const f2v>)p;
-    return make_float2(v.x, v.y);
-}
 __device__ __forceinline__ void add_global(Global<float> p, float v) {
     (void)__hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -50,6 +50,7 @@
 #include "insert.hpp"
 #include "insert_cells.hpp"
 #include "insert_gather.hpp"
+#include "inverse.hpp"
 #include "project.hpp"
 #include "project_cells.hpp"
 #include "resolve.hpp"
@@ -490,17 +491,18 @@ int ensure_final(spbp_ctx* c) {
     c->work = nullptr; c->real = nullptr; c->wkb = nullptr; c->psum = nullptr; c->pcnt = nullptr; c->mean = nullptr;
     if (c->inv) { hipfftDestroy(c->inv); c->inv = 0; }
     const int N = c->N, nx = c->nx;
-    HIPCHK(c, dmalloc(&c->work, c->nh * sizeof(float2)));
-    HIPCHK(c, dmalloc(&c->real, (size_t)N * N * N * sizeof(float)));
+    const bool own = c->own_fwd();   // the own passes' two cropped intermediates, else the half grid and N^3 reals
+    HIPCHK(c, dmalloc(&c->work, (own ? (size_t)nx * (N + nx) * c->H : c->nh) * sizeof(float2)));
+    if (!own) HIPCHK(c, dmalloc(&c->real, (size_t)N * N * N * sizeof(float)));
     std::vector<float> w;
     wkb_table(nx, N, w);
     HIPCHK(c, dmalloc(&c->wkb, w.size() * sizeof(float)));
     HIPCHK(c, hipMemcpy(c->wkb, w.data(), w.size() * sizeof(float), hipMemcpyHostToDevice));
-    const size_t nb = nblocks((size_t)nx * nx * nx);
+    const size_t nb = own ? inv_x_blocks(nx) : nblocks((size_t)nx * nx * nx);
     HIPCHK(c, dmalloc(&c->psum, nb * sizeof(double)));
     HIPCHK(c, dmalloc(&c->pcnt, nb * sizeof(unsigned)));
     HIPCHK(c, dmalloc(&c->mean, sizeof(float)));
-    if (hipfftPlan3d(&c->inv, N, N, N, HIPFFT_C2R) != HIPFFT_SUCCESS) {
+    if (!own && hipfftPlan3d(&c->inv, N, N, N, HIPFFT_C2R) != HIPFFT_SUCCESS) {
         c->inv = 0;
         return fail(c, SPBP_ERR_FFT, "hipfftPlan3d(%d) failed", N);
     }
@@ -1480,7 +1482,9 @@ constexpr unsigned FINAL_LAUNCH_BLOCKS = (1u << 31) / TPB;
 // A run of jobs one launch of each window-step kernel covers.
 struct FinalRun {
     int j0 = 0, n = 0;
-    unsigned hb = 0, vb = 0;   // half-grid and volume blocks
+    bool own = false;                          // own inverse transform (N), else hipFFT's
+    int nmax = 0;                              // its largest N
+    unsigned hb = 0, zb = 0, xb = 0, vb = 0;   // half-grid (y pass), z pass, x pass and volume blocks
 };
 
 // Records the job table's last use at scope exit, so the next call reuses the
@@ -1492,10 +1496,11 @@ struct TableUse {
 };
 
 // Normalisation, inverse transform and window steps of every round, in waves
-// (a context's buffers serve one volume per wave): per wave one normalise
-// launch over all its volumes, their inverse transforms, one window, one
-// shell-mean and one subtract launch over all of them, then SYMVOL where
-// symmetries were inserted.  The job table lives on the first round's context.
+// (a context's buffers serve one volume per wave).  Per wave and per run of
+// volumes with own transforms: the y, z and x passes (inverse.hpp), else a
+// normalise launch, hipFFT's transforms and a window launch; then a shell-mean
+// and a subtract launch, then SYMVOL where symmetries were inserted.  The job
+// table lives on the first round's context.
 int run_waves(std::vector<Round>& rs, hipStream_t st) {
     spbp_ctx* t = rs[0].c;
     int nw = 0;
@@ -1509,11 +1514,17 @@ int run_waves(std::vector<Round>& rs, hipStream_t st) {
             if (R.wave != w) continue;
             const spbp_ctx* c = R.c;
             const size_t nv = (size_t)c->nx * c->nx * c->nx;
-            const unsigned hb = (unsigned)((c->nh + (size_t)TPB * NORM_VPT - 1) / ((size_t)TPB * NORM_VPT)), vb = nblocks(nv);
+            const bool own = c->own_fwd();
+            const int slabs = own ? inv_slabs(c->N) : 0;
+            const unsigned vb = nblocks(nv), xb = own ? inv_x_blocks(c->nx) : 0, zb = (unsigned)c->nx * slabs;
+            const unsigned hb = own ? (unsigned)c->N * slabs
+                                    : (unsigned)((c->nh + (size_t)TPB * NORM_VPT - 1) / ((size_t)TPB * NORM_VPT));
             auto& rw = runs[w];
-            if (rw.empty() || (unsigned long long)rw.back().hb + hb > FINAL_LAUNCH_BLOCKS ||
-                (unsigned long long)rw.back().vb + vb > FINAL_LAUNCH_BLOCKS) {
+            const unsigned long long lim = FINAL_LAUNCH_BLOCKS / (INV_NT / TPB);   // a block has up to INV_NT threads
+            if (rw.empty() || rw.back().own != own || rw.back().hb + (unsigned long long)hb > lim ||
+                rw.back().xb + (unsigned long long)xb > lim || rw.back().vb + (unsigned long long)vb > lim) {
                 FinalRun fr;
+                fr.own = own;
                 fr.j0 = (int)fj.size();
                 rw.push_back(fr);
             }
@@ -1534,9 +1545,18 @@ int run_waves(std::vector<Round>& rs, hipStream_t st) {
             f.invN = 1.0 / c->N;
             f.invL = 1.0 / c->nx;
             f.hb0 = fr.hb;
+            f.zb0 = fr.zb;
+            f.xb0 = fr.xb;
             f.vb0 = fr.vb;
-            f.vnb = vb;
+            f.vnb = own ? xb : vb;
+            f.slabs = slabs;
+            f.pairs = own ? inv_pairs(c->nx) : 0;
+            f.tw = c->tw;
+            f.fft = own ? fft_plan(c->N) : FftPlan{};
+            fr.nmax = std::max(fr.nmax, c->N);
             fr.hb += hb;
+            fr.zb += zb;
+            fr.xb += xb;
             fr.vb += vb;
             ++fr.n;
             fj.push_back(f);
@@ -1560,15 +1580,27 @@ int run_waves(std::vector<Round>& rs, hipStream_t st) {
     TableUse use{t, st};
     HIPCHK(t, hipMemcpyAsync(t->fjobs_d, t->fjobs_h, n * sizeof(FinalJob), hipMemcpyHostToDevice, st));
     for (int w = 0; w < nw; ++w) {
-        for (const FinalRun& fr : runs[w]) normalize_kernel<<<fr.hb, TPB, 0, st>>>(t->fjobs_d + fr.j0, fr.n);
-        HIPCHK(t, hipGetLastError());
+        for (const FinalRun& fr : runs[w]) {
+            if (fr.own) continue;
+            normalize_kernel<<<fr.hb, TPB, 0, st>>>(t->fjobs_d + fr.j0, fr.n);
+            HIPCHK(t, hipGetLastError());
+        }
         for (int i : members[w]) {
             spbp_ctx* c = rs[i].c;
+            if (c->own_fwd()) continue;
             FFTCHK(c, hipfftSetStream(c->inv, st));
             FFTCHK(c, hipfftExecC2R(c->inv, (hipfftComplex*)c->work, (hipfftReal*)c->real));
         }
         for (const FinalRun& fr : runs[w]) {
-            window_kernel<<<fr.vb, TPB, 0, st>>>(t->fjobs_d + fr.j0, fr.n);
+            const FinalJob* jobs = t->fjobs_d + fr.j0;
+            if (fr.own) {
+                const size_t tw = fr.nmax * sizeof(float2);
+                inv_y_kernel<<<fr.hb, INV_NT, tw, st>>>(jobs, fr.n);
+                inv_z_kernel<<<fr.zb, INV_NT, tw, st>>>(jobs, fr.n);
+                inv_x_kernel<<<fr.xb, TPB, tw, st>>>(jobs, fr.n);
+            } else {
+                window_kernel<<<fr.vb, TPB, 0, st>>>(jobs, fr.n);
+            }
             shell_mean_kernel<<<fr.n, TPB, 0, st>>>(t->fjobs_d + fr.j0);
             subtract_kernel<<<fr.vb, TPB, 0, st>>>(t->fjobs_d + fr.j0, fr.n);
         }
