@@ -1,7 +1,7 @@
 // finalize.hpp -- SYMPLANE0 / NRMW2 / WINDKB2A kernels and partial volumes.
 #pragma once
 #include "common.hpp"
-#include "fft_any.hpp"
+#include "fft.hpp"
 
 namespace spbp {
 

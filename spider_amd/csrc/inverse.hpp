@@ -15,7 +15,7 @@
 // into a full half grid, hipFFT's 3D transform with its transposes and a window
 // pass over N^3 reals moved over three times as much, and a context's plan cost
 // ~5 ms to make and ~5 ms to destroy.  Three volumes of two halves, before and
-// after: 256^3 into 128^3 0.93 -> 0.29 ms; a context of 64^3 from 300
+// after: 256^3 into 128^3 0.93 -> 0.25 ms; a context of 64^3 from 300
 // projections, made, used and destroyed: 10.7 -> 1.8 ms.
 //
 // y before z: the accumulators' rows of a plane are N / 2 + 1 values apart, those
@@ -31,18 +31,9 @@
 // transform uses the Hermitian parts only; their transform along y and z is the
 // real part of the planes' own, which is what the x pass reads.
 #pragma once
-#include "fft_any.hpp"
 #include "finalize.hpp"
 
 namespace spbp {
-
-// Blocks go round the eight XCDs in turn; work item `order` gives each XCD a
-// contiguous range, so neighbouring slabs, whose rows share cache lines at
-// their unaligned ends, meet in one L2.
-__device__ __forceinline__ unsigned xcd_order(unsigned b, unsigned n) {
-    const unsigned q = n >> 3, r = n & 7, x = b & 7;
-    return x * q + min(x, r) + (b >> 3);
-}
 
 struct Slab {
     int row, c0, cw, lc;   // lc: log2 of the power of two >= cw
@@ -60,6 +51,7 @@ __device__ __forceinline__ Slab slab_of(unsigned w, int slabs, int H) {
 // Element (n, m) of a slab: row n, column m; a thread keeps its column, and its
 // rows are n0, n0 + dn, ...  Columns m >= cw idle (they load a column that exists).
 
+template <bool P2>
 __global__ __launch_bounds__(INV_NT) void inv_y_kernel(const FinalJob* __restrict__ jobs, int nj) {
     __shared__ float2 buf[INV_LDS];
     extern __shared__ float2 stw[];
@@ -140,12 +132,13 @@ __global__ __launch_bounds__(INV_NT) void inv_y_kernel(const FinalJob* __restric
         }
     }
     __syncthreads();
-    any_fft<INV_ELEMS, INV_NT>(buf, s.cw, p, S, stw);
+    lds_fft<INV_ELEMS, INV_NT, P2>(buf, s.cw, p, S, stw);
     const Global<float2> out = as_global(f.work) + (size_t)k * nx * H;
     if (m < s.cw)
         for (int y = n0; y < nx; y += dn) store2(out + (unsigned)(y * H + i), buf[m * S + ip + y]);
 }
 
+template <bool P2>
 __global__ __launch_bounds__(INV_NT) void inv_z_kernel(const FinalJob* __restrict__ jobs, int nj) {
     __shared__ float2 buf[INV_LDS];
     extern __shared__ float2 stw[];
@@ -168,18 +161,19 @@ __global__ __launch_bounds__(INV_NT) void inv_z_kernel(const FinalJob* __restric
             if (nb + u * dn < N && m < s.cw) buf[m * S + nb + u * dn] = v[u];
     }
     __syncthreads();
-    any_fft<INV_ELEMS, INV_NT>(buf, s.cw, p, S, stw);
+    lds_fft<INV_ELEMS, INV_NT, P2>(buf, s.cw, p, S, stw);
     const Global<float2> out = as_global(f.work) + (size_t)nx * N * H + (size_t)s.row * H + s.c0 + m;
     if (m < s.cw)
         for (int z = n0; z < nx; z += dn) store2(out + (size_t)z * pitch, buf[m * S + ip + z]);
 }
 
+template <bool P2>
 __global__ __launch_bounds__(TPB) void inv_x_kernel(const FinalJob* __restrict__ jobs, int nj) {
-    __shared__ float2 buf[FFT_ROW_ELEMS];
+    __shared__ float2 buf[FFT_ROW_LDS];
     extern __shared__ float2 stw[];
     const FinalJob& f = jobs[job_of_block<2>(jobs, nj, blockIdx.x)];
     const FftPlan& p = f.fft;
-    const int nx = f.nx, N = f.N, H = nx + 1, ip = (N - nx) / 2 + (nx % 2);
+    const int nx = f.nx, N = f.N, H = nx + 1, S = N + 1, ip = (N - nx) / 2 + (nx % 2);
     const unsigned lb = blockIdx.x - f.xb0;
     for (int i = threadIdx.x; i < N; i += TPB) stw[i] = f.tw[i];
     const int rows = nx * nx, M = f.pairs, r0 = 2 * M * (int)lb, mc = min(M, (rows - r0 + 1) / 2);
@@ -200,15 +194,15 @@ __global__ __launch_bounds__(TPB) void inv_x_kernel(const FinalJob* __restrict__
             if (idx >= mc * H) continue;
             const int m = div_by(idx, p.mH), i = idx - m * H;
             if (i == 0 || i == nx) {
-                buf[m * N + i] = make_float2(a[u].x, b[u].x);
+                buf[m * S + i] = make_float2(a[u].x, b[u].x);
             } else {
-                buf[m * N + i] = make_float2(a[u].x - b[u].y, a[u].y + b[u].x);
-                buf[m * N + N - i] = make_float2(a[u].x + b[u].y, b[u].x - a[u].y);
+                buf[m * S + i] = make_float2(a[u].x - b[u].y, a[u].y + b[u].x);
+                buf[m * S + N - i] = make_float2(a[u].x + b[u].y, b[u].x - a[u].y);
             }
         }
     }
     __syncthreads();
-    any_fft<FFT_ROW_ELEMS, TPB>(buf, mc, p, N, stw);
+    lds_fft<FFT_ROW_ELEMS, TPB, P2>(buf, mc, p, S, stw);
     double sum = 0.0;
     unsigned cnt = 0;
     const int cc = nx / 2, nr = min(2 * mc, rows - r0);
@@ -216,7 +210,7 @@ __global__ __launch_bounds__(TPB) void inv_x_kernel(const FinalJob* __restrict__
     const Global<float> out = as_global(f.out) + (size_t)r0 * nx;
     for (int idx = threadIdx.x; idx < nr * nx; idx += TPB) {
         const int q = div_by(idx, p.mL), x = idx - q * nx, r = r0 + q, z = r / nx, y = r - z * nx;
-        const float2 t = buf[(q >> 1) * N + ip + x];
+        const float2 t = buf[(q >> 1) * S + ip + x];
         float v = (q & 1 ? t.y : t.x) * f.pix;   // FMRS_3 scale
         const int lr = (x - cc) * (x - cc) + (y - cc) * (y - cc) + (z - cc) * (z - cc);
         if (lr <= cc * cc) {

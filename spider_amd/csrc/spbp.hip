@@ -44,7 +44,6 @@
 #include "calib.hpp"
 #include "common.hpp"
 #include "fft.hpp"
-#include "fft_any.hpp"
 #include "finalize.hpp"
 #include "hostmath.hpp"
 #include "insert.hpp"
@@ -139,9 +138,9 @@ struct spbp_ctx {
     int c2r_cap = 0;
     // own forward transforms (power-of-two N): e^{-2 pi i m / N}, m < N
     float2* tw = nullptr;
-    int fft_log2 = 0;   // log2 N of a power of two the own transforms take, else 0
-    FftPlan fft{};      // the own transforms' passes for other N = 2^a 3^b 5^c 7^d (np > 0)
-    bool own_fwd() const { return fft_log2 > 0 || fft.np > 0; }   // else hipFFT does the forward transforms
+    FftPlan fft{};      // the own transforms' passes (N = 2^a 3^b 5^c 7^d), or np = 0: hipFFT's
+    bool own_fwd() const { return fft.np > 0; }
+    bool pow2() const { return own_fwd() && (N & (N - 1)) == 0; }
     double* fmean = nullptr;   // per chunk image: PADD2's mean
     // finalisation
     hipfftHandle inv = 0;
@@ -815,9 +814,10 @@ int run_insert(spbp_ctx* c, int img0, const Geom* geom_d, int ng, const Targets&
 // The own two-pass R2C of b zero-padded images minus c->fmean[i] into c->spec; c->vmax receives each spectrum's largest |Re|, |Im| and
 // must be zero on entry.
 int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
-    const size_t lds = fft_lds_bytes(c->N), rlds = fft_lds_bytes(c->N, FFT_ROW_ELEMS);
+    const size_t lds = fft_lds_bytes(c->N, FFT_LDS), rlds = fft_lds_bytes(c->N, FFT_ROW_LDS);
     const int pairs = (c->nx + 1) / 2, M = std::min(FFT_ROW_ELEMS / c->N, pairs);   // >= 1: own transforms need N <= FFT_ROW_ELEMS
-    const int cw = FFT_ELEMS / c->N;
+    const int cmax = FFT_ELEMS / c->N, width = (c->nx + (c->nx + cmax - 1) / cmax - 1) / ((c->nx + cmax - 1) / cmax);
+    const int slabs = (c->nx + width - 1) / width;   // equal slabs, but the last
     const size_t npix = (size_t)c->nx * c->nx, nspec = (size_t)c->N * c->H;
     const size_t esz = dtype == SPBP_BF16 ? 2 : 4;
     // sub-batches whose row-pass output (~256 MiB, the size of MI355X's
@@ -833,24 +833,16 @@ int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
         {
             Timed tm(c, SPBP_K_PAD, n, st);
             const dim3 rgrid((pairs + M - 1) / M, n);
-            if (!c->fft_log2 && dtype == SPBP_BF16)
-                row_any_kernel<uint16_t><<<rgrid, TPB, rlds, st>>>((const uint16_t*)im, c->nx, c->fft, c->tw, c->fmean + s0, sp);
-            else if (!c->fft_log2)
-                row_any_kernel<float><<<rgrid, TPB, rlds, st>>>((const float*)im, c->nx, c->fft, c->tw, c->fmean + s0, sp);
-            else if (dtype == SPBP_BF16)
-                row_fft_kernel<uint16_t><<<rgrid, TPB, rlds, st>>>((const uint16_t*)im, c->nx, c->N, c->fft_log2, c->tw,
-                                                                  c->fmean + s0, sp);
+            const auto args = [&](auto kernel, auto* p) { kernel<<<rgrid, TPB, rlds, st>>>(p, c->nx, c->fft, c->tw, c->fmean + s0, sp); };
+            if (dtype == SPBP_BF16)
+                args(c->pow2() ? row_fft_kernel<uint16_t, true> : row_fft_kernel<uint16_t, false>, (const uint16_t*)im);
             else
-                row_fft_kernel<float><<<rgrid, TPB, rlds, st>>>((const float*)im, c->nx, c->N, c->fft_log2, c->tw,
-                                                               c->fmean + s0, sp);
+                args(c->pow2() ? row_fft_kernel<float, true> : row_fft_kernel<float, false>, (const float*)im);
         }
         {
             Timed tm(c, SPBP_K_FFT2, n, st);
-            const dim3 cgrid((c->H + cw - 1) / cw, n);
-            if (c->fft_log2)
-                col_fft_kernel<<<cgrid, FFT_COL_NT, lds, st>>>(c->nx, c->N, c->fft_log2, c->tw, sp, c->vmax + s0);
-            else
-                col_any_kernel<<<cgrid, FFT_COL_NT, lds, st>>>(c->nx, c->fft, c->tw, sp, c->vmax + s0);
+            const auto kernel = c->pow2() ? col_fft_kernel<true> : col_fft_kernel<false>;
+            kernel<<<(unsigned)(n * slabs), FFT_COL_NT, lds, st>>>(c->nx, c->fft, slabs, width, c->tw, sp, c->vmax + s0);
         }
     }
     HIPCHK(c, hipGetLastError());
@@ -859,20 +851,16 @@ int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
 
 int pad_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
     if (c->own_fwd()) {
-        if (!c->fft_log2) {
+        if (!c->pow2()) {
             int rc = tail_ok(c, b);
             if (rc) return rc;
         }
         {
             Timed tm(c, SPBP_K_PAD, b, st);   // the means of the whole chunk (one block per image)
-            if (!c->fft_log2 && dtype == SPBP_BF16)
-                pad_mean_any_kernel<uint16_t><<<b, TPB, 0, st>>>((const uint16_t*)src, c->nx, c->fmean, c->vmax);
-            else if (!c->fft_log2)
-                pad_mean_any_kernel<float><<<b, TPB, 0, st>>>((const float*)src, c->nx, c->fmean, c->vmax);
-            else if (dtype == SPBP_BF16)
-                pad_mean_kernel<uint16_t><<<b, TPB, 0, st>>>((const uint16_t*)src, c->nx, c->fft_log2 - 1, c->fmean, c->vmax);
+            if (dtype == SPBP_BF16)
+                pad_mean_kernel<uint16_t><<<b, TPB, 0, st>>>((const uint16_t*)src, c->nx, c->fft.mL, c->fmean, c->vmax);
             else
-                pad_mean_kernel<float><<<b, TPB, 0, st>>>((const float*)src, c->nx, c->fft_log2 - 1, c->fmean, c->vmax);
+                pad_mean_kernel<float><<<b, TPB, 0, st>>>((const float*)src, c->nx, c->fft.mL, c->fmean, c->vmax);
         }
         return own_fft(c, src, dtype, b, st);
     }
@@ -1482,7 +1470,7 @@ constexpr unsigned FINAL_LAUNCH_BLOCKS = (1u << 31) / TPB;
 // A run of jobs one launch of each window-step kernel covers.
 struct FinalRun {
     int j0 = 0, n = 0;
-    bool own = false;                          // own inverse transform (N), else hipFFT's
+    bool own = false, p2 = true;               // own inverse transforms, all of them powers of two; else hipFFT's
     int nmax = 0;                              // its largest N
     unsigned hb = 0, zb = 0, xb = 0, vb = 0;   // half-grid (y pass), z pass, x pass and volume blocks
 };
@@ -1552,8 +1540,9 @@ int run_waves(std::vector<Round>& rs, hipStream_t st) {
             f.slabs = slabs;
             f.pairs = own ? inv_pairs(c->nx) : 0;
             f.tw = c->tw;
-            f.fft = own ? fft_plan(c->N) : FftPlan{};
+            f.fft = c->fft;
             fr.nmax = std::max(fr.nmax, c->N);
+            fr.p2 = fr.p2 && c->pow2();
             fr.hb += hb;
             fr.zb += zb;
             fr.xb += xb;
@@ -1595,9 +1584,9 @@ int run_waves(std::vector<Round>& rs, hipStream_t st) {
             const FinalJob* jobs = t->fjobs_d + fr.j0;
             if (fr.own) {
                 const size_t tw = fr.nmax * sizeof(float2);
-                inv_y_kernel<<<fr.hb, INV_NT, tw, st>>>(jobs, fr.n);
-                inv_z_kernel<<<fr.zb, INV_NT, tw, st>>>(jobs, fr.n);
-                inv_x_kernel<<<fr.xb, TPB, tw, st>>>(jobs, fr.n);
+                (fr.p2 ? inv_y_kernel<true> : inv_y_kernel<false>)<<<fr.hb, INV_NT, tw, st>>>(jobs, fr.n);
+                (fr.p2 ? inv_z_kernel<true> : inv_z_kernel<false>)<<<fr.zb, INV_NT, tw, st>>>(jobs, fr.n);
+                (fr.p2 ? inv_x_kernel<true> : inv_x_kernel<false>)<<<fr.xb, TPB, tw, st>>>(jobs, fr.n);
             } else {
                 window_kernel<<<fr.vb, TPB, 0, st>>>(jobs, fr.n);
             }
@@ -1730,8 +1719,7 @@ int spbp_create(const spbp_opts* o, spbp_ctx** out) {
         // list builds and fewer persistent-kernel tails: 20,000 projections
         // of 128^2 go through one launch (481.8k proj/s for a BP 32F job,
         // 473.5k in three launches of 2 GiB chunks).
-        const bool own = (c->N & (c->N - 1)) == 0 && c->N >= 8 && c->N <= std::min(2048, FFT_ROW_ELEMS) &&
-                         !(o->flags & SPBP_HIPFFT);
+        const bool own = fft_plan(c->N).np && !(o->flags & SPBP_HIPFFT);
         const size_t per = (own ? 0 : (size_t)c->N * c->N * 4) + (size_t)c->N * c->H * 8;
         c->batch = (int)std::max<size_t>(16, std::min<size_t>(32768, ((size_t)8192 << 20) / per));
     }
@@ -1779,10 +1767,7 @@ int spbp_create(const spbp_opts* o, spbp_ctx** out) {
         if (dmalloc(&c->tw, t.size() * sizeof(float2)) != hipSuccess ||
             hipMemcpy(c->tw, t.data(), t.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess)
             return bail(fail(nullptr, SPBP_ERR_ALLOC, "twiddle table"));
-        if ((c->N & (c->N - 1)) == 0)
-            while ((1 << c->fft_log2) < c->N) ++c->fft_log2;
-        else
-            c->fft = fp;
+        c->fft = fp;
     }
     // default plan: owner-computes bricks of unit cells (by nearest voxel in launches with few sections), 128
     // projections per item: fastest measured at 128^2 into 256^3 and 256^2 into 512^3; spbp_tune picks per workload
@@ -1969,7 +1954,7 @@ int spbp_scatter_images(spbp_ctx* c, const float* imgs, int nimg, const double* 
     if (nimg < 0) return fail(c, SPBP_ERR_ARG, "negative projection count %d", nimg);
     if (nimg == 0) return SPBP_OK;
     if (!imgs || !X) return fail(c, SPBP_ERR_ARG, "NULL image or grid pointer");
-    if (!c->fft_log2) return fail(c, SPBP_ERR_SIZE, "the image adjoint needs a power-of-two padded size (N = %d)", c->N);
+    if (!c->pow2()) return fail(c, SPBP_ERR_SIZE, "the image adjoint needs a power-of-two padded size (N = %d)", c->N);
     DeviceGuard dg(c->device);
     hipStream_t st = (hipStream_t)stream;
     int rc = stage_geom(c, nimg, dm, angles_deg, nullptr, st, false);
