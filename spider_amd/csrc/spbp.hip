@@ -1372,7 +1372,7 @@ int phase_term_counts(Round& R, hipStream_t st) {
         (rc = launch_hits<1>(R, 2 * R.nv * R.nchunks, st)))
         return rc;
     if (R.nhits > 0)
-        term_kernel<P, false><<<(unsigned)((R.nhits + RES_TPB - 1) / RES_TPB), RES_TPB, 0, st>>>(
+        term_kernel<P, false><<<term_blocks(R.nhits), RES_TPB, 0, st>>>(
             r.hits, R.nhits, r.list, c->hist_d, res_table<P>(c), res_fltb<P>(c), c->nx, c->N, r.tcnt, nullptr, nullptr);
     if ((rc = scan_counts(c, r, r.tcnt, R.nhits, r.toff, st))) return rc;
     HIPCHK(c, hipMemcpyAsync(r.h, r.toff + R.nhits, sizeof(long long), hipMemcpyDeviceToHost, st));
@@ -1391,7 +1391,7 @@ int phase_decide(Round& R, double* wout, hipStream_t st) {
         (rc = grow(c, r.sums, r.sums_cap, (size_t)nitems * 2 * sizeof(P), "weight sums")))
         return rc;
     if (R.nhits > 0)
-        term_kernel<P, true><<<(unsigned)((R.nhits + RES_TPB - 1) / RES_TPB), RES_TPB, 0, st>>>(
+        term_kernel<P, true><<<term_blocks(R.nhits), RES_TPB, 0, st>>>(
             r.hits, R.nhits, r.list, c->hist_d, res_table<P>(c), res_fltb<P>(c), c->nx, c->N, nullptr, r.toff,
             (P*)r.terms);
     sum_kernel<P><<<(unsigned)((nitems + RES_TPB - 1) / RES_TPB), RES_TPB, 0, st>>>(nitems, R.nchunks, r.off, r.toff,
