@@ -3,6 +3,7 @@
 // BI-layout spectra go through the insertion kernels.
 #pragma once
 #include "common.hpp"
+#include "fft.hpp"
 
 namespace spbp {
 
@@ -136,8 +137,98 @@ __global__ __launch_bounds__(GT * GT) void gather_kernel(const float2* __restric
     *o = make_float2((float)re, (float)(flip ? -im : im));
 }
 
-// The projector's image synthesis from gathered BI spectra, before the C2R
-// transform: in place, C(I, jp) = conj(BI(I, jp) (-1)^(I + jp)), and column 0
+// ------------------------------------------------------------------ image synthesis
+// images = crop(irfft2(C)), C(I, jp) = conj(BI(I, jp) (-1)^(I + jp)) with column 0
+// completed by Hermitian symmetry, as the forward transform of conj(C), which
+// has the same real sum: synth_col_kernel transforms slabs of columns and keeps
+// the NX rows of the crop (in place: rows 0 .. NX - 1), synth_row_kernel makes
+// one complex transform of two rows' half spectra and writes their crop.  Of
+// columns 0 and N/2 the row transform uses the real parts.
+//
+// Bound by memory: N rows read, NX written and read, NX rows of pixels written.
+// hipFFT transformed and stored all N rows, after a pass that completed the
+// spectra and before one that cropped: 4,096 images of 128^2 1.92 ms, here 0.56.
+template <bool P2>
+__global__ __launch_bounds__(FFT_COL_NT) void synth_col_kernel(int nx, FftPlan p, int slabs, int width,
+                                                               const float2* __restrict__ tw, float2* __restrict__ spec) {
+    extern __shared__ float2 lds[];
+    float2* buf = lds;
+    float2* stw = lds + FFT_LDS;
+    const int N = p.N, H = nx + 1, S = N + 1, ip = (N - nx) / 2 + (nx % 2);
+    load_twiddles(stw, tw, N);
+    const unsigned w = xcd_order(blockIdx.x, gridDim.x), b = w / (unsigned)slabs;
+    const int c0 = (int)(w - b * (unsigned)slabs) * width, cw = min(width, H - c0);
+    float2* sp = spec + (size_t)b * N * H + c0;
+    const int lc = cw > 1 ? 32 - __clz(cw - 1) : 0, cp = 1 << lc;
+    const int m = threadIdx.x & (cp - 1), n0 = threadIdx.x >> lc, dn = FFT_COL_NT >> lc;
+    if (m < cw) {
+        for (int nb = n0; nb < N; nb += FFT_BATCH * dn) {
+            float2 v[FFT_BATCH];
+#pragma unroll
+            for (int u = 0; u < FFT_BATCH; ++u) {
+                const int n = min(nb + u * dn, N - 1);
+                v[u] = sp[(c0 + m == 0 && n > nx ? N - n : n) * H + m];
+            }
+#pragma unroll
+            for (int u = 0; u < FFT_BATCH; ++u) {
+                const int n = nb + u * dn;
+                const float sg = ((c0 + m + n) & 1) ? -1.0f : 1.0f;   // N is even: the mirror row has the same sign
+                if (n < N) buf[m * S + n] = make_float2(v[u].x * sg, c0 + m == 0 && n > nx ? -(v[u].y * sg) : v[u].y * sg);
+            }
+        }
+    }
+    __syncthreads();
+    lds_fft<FFT_ELEMS, FFT_COL_NT, P2>(buf, cw, p, S, stw);
+    if (m < cw)
+        for (int n = n0; n < nx; n += dn) sp[n * H + m] = buf[m * S + ip + n];
+}
+
+// Block per (image, group of FFT_ROW_ELEMS / N row pairs).
+template <bool P2>
+__global__ __launch_bounds__(TPB) void synth_row_kernel(int nx, FftPlan p, const float2* __restrict__ tw,
+                                                        const float2* __restrict__ spec, float* __restrict__ imgs) {
+    extern __shared__ float2 lds[];
+    float2* buf = lds;
+    float2* stw = lds + FFT_ROW_LDS;
+    const int N = p.N, H = nx + 1, S = N + 1, ip = (N - nx) / 2 + (nx % 2);
+    load_twiddles(stw, tw, N);
+    const int pairs = (nx + 1) / 2, M = min(FFT_ROW_ELEMS / N, pairs);
+    const int p0 = blockIdx.x * M, mc = min(M, pairs - p0), nr = min(2 * mc, nx - 2 * p0);
+    const float2* in = spec + (size_t)blockIdx.y * N * H + (size_t)2 * p0 * H;
+    constexpr int U = FFT_BATCH / 2;
+    for (int i0 = threadIdx.x; i0 < mc * H; i0 += U * TPB) {
+        float2 a[U], b[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int idx = min(i0 + u * TPB, mc * H - 1), m = div_by(idx, p.mH), i = idx - m * H;
+            a[u] = in[2 * m * H + i];
+            b[u] = in[min(2 * m + 1, nr - 1) * H + i];   // odd NX: the last row pairs with itself
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int idx = i0 + u * TPB;
+            if (idx >= mc * H) continue;
+            const int m = div_by(idx, p.mH), i = idx - m * H;
+            if (i == 0 || i == nx) {
+                buf[m * S + i] = make_float2(a[u].x, b[u].x);
+            } else {
+                buf[m * S + i] = make_float2(a[u].x - b[u].y, a[u].y + b[u].x);
+                buf[m * S + N - i] = make_float2(a[u].x + b[u].y, b[u].x - a[u].y);
+            }
+        }
+    }
+    __syncthreads();
+    lds_fft<FFT_ROW_ELEMS, TPB, P2>(buf, mc, p, S, stw);
+    const float inv = 1.0f / (float)((double)N * (double)N);   // the inverse transform's normalisation
+    float* out = imgs + (size_t)blockIdx.y * nx * nx + (size_t)2 * p0 * nx;
+    for (int idx = threadIdx.x; idx < nr * nx; idx += TPB) {
+        const int q = div_by(idx, p.mL), x = idx - q * nx;
+        const float2 t = buf[(q >> 1) * S + ip + x];
+        out[idx] = (q & 1 ? t.y : t.x) * inv;
+    }
+}
+
+// The same through hipFFT, for other N: before the C2R transform, in place, C(I, jp) = conj(BI(I, jp) (-1)^(I + jp)), and column 0
 // completed by Hermitian symmetry, C(0, N - jp) = conj(C(0, jp)) for
 // 0 < jp < NX (the rows J < 0 of column 0 are not gathered).  One thread per
 // entry; column 0's pairs by the thread of jp.

@@ -1912,6 +1912,21 @@ int spbp_gather_images(spbp_ctx* c, const float* X, int nimg, const double* angl
     if (rc) return rc;
     if ((rc = ensure_chunk(c, std::min(c->batch, nimg)))) return rc;
     const int N = c->N, H = c->H, B = c->fwd_batch;
+    if (c->own_fwd()) {
+        const int cmax = FFT_ELEMS / N, width = (H + (H + cmax - 1) / cmax - 1) / ((H + cmax - 1) / cmax);
+        const int slabs = (H + width - 1) / width, pairs = (c->nx + 1) / 2, M = std::min(FFT_ROW_ELEMS / N, pairs);
+        const size_t lds = fft_lds_bytes(N, FFT_LDS), rlds = fft_lds_bytes(N, FFT_ROW_LDS);
+        for (int p0 = 0; p0 < nimg; p0 += B) {
+            const int b = std::min(B, nimg - p0);
+            if ((rc = launch_slices(c, (const float2*)X, c->geom_d + p0, p0, b, c->spec, st))) return rc;
+            (c->pow2() ? synth_col_kernel<true> : synth_col_kernel<false>)<<<(unsigned)(b * slabs), FFT_COL_NT, lds, st>>>(
+                c->nx, c->fft, slabs, width, c->tw, c->spec);
+            (c->pow2() ? synth_row_kernel<true> : synth_row_kernel<false>)<<<dim3((pairs + M - 1) / M, b), TPB, rlds, st>>>(
+                c->nx, c->fft, c->tw, c->spec, imgs + (size_t)p0 * c->nx * c->nx);
+            HIPCHK(c, hipGetLastError());
+        }
+        return SPBP_OK;
+    }
     if (c->c2r_cap < B) {
         c->c2r_cap = 0;
         if (c->c2rbuf) { (void)hipFree(c->c2rbuf); c->c2rbuf = nullptr; }
