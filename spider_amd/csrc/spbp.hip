@@ -810,10 +810,10 @@ int run_insert(spbp_ctx* c, int img0, const Geom* geom_d, int ng, const Targets&
     return launch_bricks(c, &job, 1, c->bnext, st, t.W0 != nullptr || t.W1 != nullptr, few);
 }
 
-// PADD2 + batched forward FFT of b images into c->spec.
-// The own two-pass R2C of b zero-padded images minus c->fmean[i] into c->spec; c->vmax receives each spectrum's largest |Re|, |Im| and
-// must be zero on entry.
-int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
+// The own two-pass R2C of b zero-padded images minus c->fmean[i] into c->spec,
+// or (adjoint) the values the projector's adjoint inserts; c->vmax receives each
+// spectrum's largest |Re|, |Im| and must be zero on entry.
+int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st, bool adjoint = false) {
     const size_t lds = fft_lds_bytes(c->N, FFT_LDS), rlds = fft_lds_bytes(c->N, FFT_ROW_LDS);
     const int pairs = (c->nx + 1) / 2, M = std::min(FFT_ROW_ELEMS / c->N, pairs);   // >= 1: own transforms need N <= FFT_ROW_ELEMS
     const int cmax = FFT_ELEMS / c->N, width = (c->nx + (c->nx + cmax - 1) / cmax - 1) / ((c->nx + cmax - 1) / cmax);
@@ -841,7 +841,8 @@ int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
         }
         {
             Timed tm(c, SPBP_K_FFT2, n, st);
-            const auto kernel = c->pow2() ? col_fft_kernel<true> : col_fft_kernel<false>;
+            const auto kernel = adjoint ? (c->pow2() ? col_fft_kernel<true, true> : col_fft_kernel<false, true>)
+                                        : (c->pow2() ? col_fft_kernel<true, false> : col_fft_kernel<false, false>);
             kernel<<<(unsigned)(n * slabs), FFT_COL_NT, lds, st>>>(c->nx, c->fft, slabs, width, c->tw, sp, c->vmax + s0);
         }
     }
@@ -849,6 +850,7 @@ int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
     return SPBP_OK;
 }
 
+// PADD2 + batched forward FFT of b images into c->spec.
 int pad_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
     if (c->own_fwd()) {
         if (!c->pow2()) {
@@ -1975,20 +1977,15 @@ int spbp_scatter_images(spbp_ctx* c, const float* imgs, int nimg, const double* 
     int rc = stage_geom(c, nimg, dm, angles_deg, nullptr, st, false);
     if (rc) return rc;
     if ((rc = ensure_chunk(c, std::min(c->batch, nimg)))) return rc;
-    const int N = c->N, H = c->H;
     const size_t npix = (size_t)c->nx * c->nx;
     const Targets t{(float2*)X, nullptr, nullptr, nullptr, nullptr, nullptr};
     for (int p0 = 0; p0 < nimg; p0 += c->fwd_batch) {
         const int b = std::min(c->fwd_batch, nimg - p0);
-        const size_t n = (size_t)b * N * H;
         // no PADD2 mean: zero means (all-zero bits are 0.0) and zero maxima
         fill((float*)c->fmean, 2 * (size_t)b, 0.0f, st);
         fill(c->vmax, b, 0.0f, st);
         HIPCHK(c, hipGetLastError());
-        if ((rc = own_fft(c, imgs + (size_t)p0 * npix, SPBP_F32, b, st))) return rc;
-        adjoint_spectrum_kernel<<<nblocks(n), TPB, 0, st>>>(c->spec, N, H, c->nx, n);
-        spec_absmax_kernel<<<b, TPB, 0, st>>>(c->spec, N * H, c->vmax);
-        HIPCHK(c, hipGetLastError());
+        if ((rc = own_fft(c, imgs + (size_t)p0 * npix, SPBP_F32, b, st, true))) return rc;
         if ((rc = run_insert(c, p0, c->geom_d + p0, b, t, st, b))) return rc;
     }
     return SPBP_OK;
