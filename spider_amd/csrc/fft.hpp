@@ -311,7 +311,7 @@ __device__ inline float4 load_img4(const uint16_t* p) {
 // image (PADD2: image minus the FP64 mean, bp3f.f:1316-1345), columns 0 ..
 // N/2 - 1, with column N/2's (real) value as the imaginary part of column 0's.
 template <typename T, bool P2>
-__global__ __launch_bounds__(TPB) void row_fft_kernel(const T* __restrict__ imgs, int nx, FftPlan p,
+__global__ __launch_bounds__(TPB) void row_fft_kernel(const T* __restrict__ imgs, int nx, FftPlan p, int groups,
                                                       const float2* __restrict__ tw, const double* __restrict__ mean,
                                                       float2* __restrict__ spec) {
     extern __shared__ float2 lds[];
@@ -319,11 +319,11 @@ __global__ __launch_bounds__(TPB) void row_fft_kernel(const T* __restrict__ imgs
     float2* stw = lds + FFT_ROW_LDS;
     const int N = p.N, H = nx + 1, S = N + 1, ip = (N - nx) / 2 + (nx % 2);
     load_twiddles(stw, tw, N);
-    const int b = blockIdx.y;
+    const unsigned b = blockIdx.x / (unsigned)groups;
     const T* img = imgs + (size_t)b * nx * nx;
     const double qs = mean[b];
     const int pairs = (nx + 1) / 2, M = min(FFT_ROW_ELEMS / N, pairs);
-    const int p0 = blockIdx.x * M, mc = min(M, pairs - p0);
+    const int p0 = (int)(blockIdx.x - b * (unsigned)groups) * M, mc = min(M, pairs - p0);
     for (int i = threadIdx.x; i < mc * nx; i += TPB) {   // the padding: N - NX = NX columns of each sequence
         const int m = div_by(i, p.mL), n = i - m * nx;
         buf[m * S + (n < ip ? n : n + nx)] = make_float2(0.f, 0.f);

@@ -185,7 +185,7 @@ __global__ __launch_bounds__(FFT_COL_NT) void synth_col_kernel(int nx, FftPlan p
 
 // Block per (image, group of FFT_ROW_ELEMS / N row pairs).
 template <bool P2>
-__global__ __launch_bounds__(TPB) void synth_row_kernel(int nx, FftPlan p, const float2* __restrict__ tw,
+__global__ __launch_bounds__(TPB) void synth_row_kernel(int nx, FftPlan p, int groups, const float2* __restrict__ tw,
                                                         const float2* __restrict__ spec, float* __restrict__ imgs) {
     extern __shared__ float2 lds[];
     float2* buf = lds;
@@ -193,8 +193,9 @@ __global__ __launch_bounds__(TPB) void synth_row_kernel(int nx, FftPlan p, const
     const int N = p.N, H = nx + 1, S = N + 1, ip = (N - nx) / 2 + (nx % 2);
     load_twiddles(stw, tw, N);
     const int pairs = (nx + 1) / 2, M = min(FFT_ROW_ELEMS / N, pairs);
-    const int p0 = blockIdx.x * M, mc = min(M, pairs - p0), nr = min(2 * mc, nx - 2 * p0);
-    const float2* in = spec + (size_t)blockIdx.y * N * H + (size_t)2 * p0 * H;
+    const unsigned img = blockIdx.x / (unsigned)groups;
+    const int p0 = (int)(blockIdx.x - img * (unsigned)groups) * M, mc = min(M, pairs - p0), nr = min(2 * mc, nx - 2 * p0);
+    const float2* in = spec + (size_t)img * N * H + (size_t)2 * p0 * H;
     constexpr int U = FFT_BATCH / 2;
     for (int i0 = threadIdx.x; i0 < mc * H; i0 += U * TPB) {
         float2 a[U], b[U];
@@ -220,7 +221,7 @@ __global__ __launch_bounds__(TPB) void synth_row_kernel(int nx, FftPlan p, const
     __syncthreads();
     lds_fft<FFT_ROW_ELEMS, TPB, P2>(buf, mc, p, S, stw);
     const float inv = 1.0f / (float)((double)N * (double)N);   // the inverse transform's normalisation
-    float* out = imgs + (size_t)blockIdx.y * nx * nx + (size_t)2 * p0 * nx;
+    float* out = imgs + (size_t)img * nx * nx + (size_t)2 * p0 * nx;
     for (int idx = threadIdx.x; idx < nr * nx; idx += TPB) {
         const int q = div_by(idx, p.mL), x = idx - q * nx;
         const float2 t = buf[(q >> 1) * S + ip + x];
@@ -260,16 +261,37 @@ __global__ __launch_bounds__(TPB) void crop_images_kernel(const float* __restric
 }
 
 // BI(I, J) -> the raw R2C value s that spectrum_value() maps to it:
-// BI = c conj(s), c = (-1)^(I + jp), so s = c conj(BI).
-__global__ __launch_bounds__(TPB) void bi_to_raw_kernel(const float2* __restrict__ bi, int N, int H, size_t n,
-                                                        float2* __restrict__ raw) {
-    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n) return;
-    const size_t r = idx % ((size_t)N * H);
-    const int jp = (int)(r / H), I = (int)(r - (size_t)jp * H);
-    const float sg = ((I + jp) & 1) ? -1.0f : 1.0f;
-    const float2 v = bi[idx];
-    raw[idx] = make_float2(v.x * sg, -v.y * sg);
+// BI = c conj(s), c = (-1)^(I + jp), so s = c conj(BI); and the spectrum's
+// largest |Re|, |Im| into vmax (zero on entry).  Block per (image, BI_BLOCK
+// values).  A pass of its own for the maxima, a block per image, took 65 us
+// for 256 spectra of 128^2.
+constexpr int BI_BLOCK = 8 * TPB;
+__global__ __launch_bounds__(TPB) void bi_to_raw_kernel(const float2* __restrict__ bi, int N, int H, unsigned blocks,
+                                                        float2* __restrict__ raw, float* __restrict__ vmax) {
+    const int per = N * H, r0 = (int)(blockIdx.x % blocks) * BI_BLOCK + threadIdx.x;
+    const unsigned b = blockIdx.x / blocks;
+    const size_t img = (size_t)b * per;
+    float2 v[BI_BLOCK / TPB];
+#pragma unroll
+    for (int u = 0; u < BI_BLOCK / TPB; ++u) v[u] = bi[img + min(r0 + u * TPB, per - 1)];
+    float m = 0.0f;
+#pragma unroll
+    for (int u = 0; u < BI_BLOCK / TPB; ++u) {
+        const int r = r0 + u * TPB;
+        if (r >= per) continue;
+        const int jp = r / H, I = r - jp * H;
+        const float sg = ((I + jp) & 1) ? -1.0f : 1.0f;
+        raw[img + r] = make_float2(v[u].x * sg, -v[u].y * sg);
+        m = fmaxf(m, fmaxf(fabsf(v[u].x), fabsf(v[u].y)));
+    }
+    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_down(m, off, 64));
+    __shared__ float sm[TPB / 64];
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < TPB / 64; ++k) m = fmaxf(m, sm[k]);
+        atomicMax((unsigned*)&vmax[b], __float_as_uint(m));   // non-negative floats order as their bits
+    }
 }
 
 }  // namespace spbp

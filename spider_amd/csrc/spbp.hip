@@ -832,8 +832,9 @@ int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st, bool
         float2* sp = c->spec + s0 * nspec;
         {
             Timed tm(c, SPBP_K_PAD, n, st);
-            const dim3 rgrid((pairs + M - 1) / M, n);
-            const auto args = [&](auto kernel, auto* p) { kernel<<<rgrid, TPB, rlds, st>>>(p, c->nx, c->fft, c->tw, c->fmean + s0, sp); };
+            const int groups = (pairs + M - 1) / M;
+            const unsigned rgrid = (unsigned)(groups * n);
+            const auto args = [&](auto kernel, auto* p) { kernel<<<rgrid, TPB, rlds, st>>>(p, c->nx, c->fft, groups, c->tw, c->fmean + s0, sp); };
             if (dtype == SPBP_BF16)
                 args(c->pow2() ? row_fft_kernel<uint16_t, true> : row_fft_kernel<uint16_t, false>, (const uint16_t*)im);
             else
@@ -1893,9 +1894,9 @@ int spbp_scatter(spbp_ctx* c, const float* bi, int nimg, const double* angles_de
     const Targets t{(float2*)X, W, nullptr, nullptr, nullptr, nullptr};
     for (int p0 = 0; p0 < nimg; p0 += c->fwd_batch) {
         const int b = std::min(c->fwd_batch, nimg - p0);
-        const size_t n = (size_t)b * N * H;
-        bi_to_raw_kernel<<<nblocks(n), TPB, 0, st>>>((const float2*)bi + (size_t)p0 * N * H, N, H, n, c->spec);
-        spec_absmax_kernel<<<b, TPB, 0, st>>>(c->spec, N * H, c->vmax);
+        fill(c->vmax, b, 0.0f, st);
+        const unsigned nbi = (unsigned)((N * H + BI_BLOCK - 1) / BI_BLOCK);
+        bi_to_raw_kernel<<<nbi * b, TPB, 0, st>>>((const float2*)bi + (size_t)p0 * N * H, N, H, nbi, c->spec, c->vmax);
         HIPCHK(c, hipGetLastError());
         if ((rc = run_insert(c, p0, c->geom_d + p0, b, t, st, b))) return rc;
     }
@@ -1923,8 +1924,8 @@ int spbp_gather_images(spbp_ctx* c, const float* X, int nimg, const double* angl
             if ((rc = launch_slices(c, (const float2*)X, c->geom_d + p0, p0, b, c->spec, st))) return rc;
             (c->pow2() ? synth_col_kernel<true> : synth_col_kernel<false>)<<<(unsigned)(b * slabs), FFT_COL_NT, lds, st>>>(
                 c->nx, c->fft, slabs, width, c->tw, c->spec);
-            (c->pow2() ? synth_row_kernel<true> : synth_row_kernel<false>)<<<dim3((pairs + M - 1) / M, b), TPB, rlds, st>>>(
-                c->nx, c->fft, c->tw, c->spec, imgs + (size_t)p0 * c->nx * c->nx);
+            (c->pow2() ? synth_row_kernel<true> : synth_row_kernel<false>)<<<(unsigned)((pairs + M - 1) / M * b), TPB, rlds, st>>>(
+                c->nx, c->fft, (pairs + M - 1) / M, c->tw, c->spec, imgs + (size_t)p0 * c->nx * c->nx);
             HIPCHK(c, hipGetLastError());
         }
         return SPBP_OK;
@@ -3005,9 +3006,9 @@ int spbp_scatter_noalloc(int nx, int flags, const float* bi, int nimg, const dou
             if (k) return fail(nullptr, SPBP_ERR_ANGLE, "rotation of image %d is not finite and orthonormal", p0 + p + 1);
         }
         HIPCHK(nullptr, hipMemcpyAsync(geom_d, gh, (size_t)b * sizeof(Geom), hipMemcpyHostToDevice, st));
-        const size_t n = (size_t)b * N * H;
-        bi_to_raw_kernel<<<nblocks(n), TPB, 0, st>>>((const float2*)bi + (size_t)p0 * N * H, N, H, n, c.spec);
-        spec_absmax_kernel<<<b, TPB, 0, st>>>(c.spec, N * H, c.vmax);
+        fill(c.vmax, b, 0.0f, st);
+        const unsigned nbi = (unsigned)((N * H + BI_BLOCK - 1) / BI_BLOCK);
+        bi_to_raw_kernel<<<nbi * b, TPB, 0, st>>>((const float2*)bi + (size_t)p0 * N * H, N, H, nbi, c.spec, c.vmax);
         HIPCHK(nullptr, hipGetLastError());
         if ((rc = build_lists(&c, geom_d, b, st, false))) return fail(nullptr, rc, "%s", c.err);
         const BrickJob job = brick_job(&c, 0, geom_d, b, t, false);
