@@ -300,7 +300,10 @@ def run_throughput(args, config, nproj, steps, warmup, op="bp32f", bf16=False, t
     avg_launch_s = ins_ms / 1e3 / launches
     per_launch = units / launches
     achieved = b_alg * per_launch / avg_launch_s / 1e9
+    # owner-computes plans take the kernel binned by unit cells from 2 NX sections per half on
+    cells = plan.get("owner_computes") and per_launch >= 2 * nx * (2 if halves else 1)
     kname = ("insert_direct_kernel" if plan["strategy"] == "direct"
+             else "insert_cells_kernel<9,9,9>" if cells
              else "insert_brick_kernel<%d,%d,%d%s>" % (*plan["brick"], ",own" if plan.get("owner_computes") else ""))
     idt = "bf16" if bf16 else "f32"
     roof = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",

@@ -55,9 +55,9 @@ extern "C" {
 #define SPBP_GEOM_F64     0x20  /* FP64 rotations (from FP64 angles), sample positions, nearest voxels
                                    and table indices: departs from the reference's fp32 geometry
                                    (oneline.f:56-105) to agree with an FP64 computation          */
-#define SPBP_HIPFFT       0x80  /* forward 2D transforms by hipFFT on the fully padded images instead
-                                   of the library's own two-pass transforms (power-of-two N only;
-                                   other sizes always use hipFFT)                              */
+#define SPBP_HIPFFT       0x80  /* transforms by hipFFT on the fully padded images and volumes
+                                   instead of the library's own cropped ones (N = 2^a 3^b 5^c 7^d
+                                   up to 2048; other sizes always use hipFFT)                  */
 #define SPBP_PLAIN_THRESHOLD 0x40 /* NRMW2's W > 0.1 test on the GPU sums alone.  By default the
                                    voxels whose W lies within 2^-11 of 0.1 are decided by
                                    re-summing their weights in the reference's order (see
@@ -142,7 +142,7 @@ int spbp_scatter_noalloc(int nx, int flags, const float* bi, int nimg, const dou
 /* The projector applied to a grid: for nimg rotations, the gather of X
  * (spbp_gather's BI spectra), completed to the full C2R input (conjugated,
  * checkerboard (-1)^(I + jp), column 0 by Hermitian symmetry), transformed
- * by hipFFT C2R, scaled by 1 / N^2 and cropped to NX x NX at the padding
+ * (own passes, or hipFFT C2R), scaled by 1 / N^2 and cropped to NX x NX at the padding
  * offset: nimg device images of NX x NX fp32.  No counterpart in the
  * reference (it has no projector matched to ONELINE). */
 int spbp_gather_images(spbp_ctx* ctx, const float* X, int nimg, const double* angles_deg, const float* dm,
@@ -198,9 +198,9 @@ typedef struct {
  * re-summation of every volume in shared phases (three host synchronisations
  * per call, four when a band list outgrows its buffer, instead of four per
  * volume), then per wave -- the first requested volume of every context,
- * then the second, then the third -- one normalisation launch over all the
- * wave's volumes, their inverse 3D transforms, and one window, shell-mean and
- * subtraction launch over all of them.  The reference finalises one volume
+ * then the second, then the third -- one launch of each pass of the inverse
+ * transform, the shell mean and the subtraction over all the wave's volumes
+ * (hipFFT's transforms are per volume).  The reference finalises one volume
  * after another (bp32f.f:275-410).  spbp_finalize is this call with one job.
  * With SPBP_TIMING each context records the call's re-summation and
  * finalisation spans.  No counterpart in the reference (one operation, one

@@ -652,7 +652,7 @@ def finalize_batch(items, full=True, halves=False, device=None) -> list:
     (spbp_finalize_batch): the threshold re-summation of all volumes shares
     its host synchronisations, and each wave of volumes -- every context's
     first requested volume, then the second, then the third -- takes one
-    normalisation and one window launch.  items: Backprojectors (finalised
+    launch of each pass.  items: Backprojectors (finalised
     with `full` / `halves`) or (Backprojector, full, halves) tuples.
     Returns one finalize()-style dict per context."""
     ctxs, outs = [], []

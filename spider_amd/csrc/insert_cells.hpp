@@ -168,7 +168,7 @@ __device__ __forceinline__ void cell_taps(Lds& L, const P (*g)[6], const unsigne
         vx[k] = (double)v[k].x * vscale;
         vy[k] = (double)v[k].y * vscale;
     }
-    // one z layer at a time (rolled: its weights are looked up here, which keeps the registers below 128)
+    // one z layer at a time (rolled: its weights are looked up here; unrolled, the registers would not fit 768 threads)
     int z8 = Lds::zpart(zl) * 8;
     P pz = (P)(z0 - 1 + zl);
 #pragma unroll 1

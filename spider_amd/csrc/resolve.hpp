@@ -11,7 +11,7 @@
 // (oneline.f:56-152).  For every voxel whose GPU weight lies in a narrow band
 // around 0.1, these kernels recompute that exact sequence from the context's
 // insertion history and record the reference's decision in a byte mask that
-// normalize_kernel reads (two bits per volume of the context):
+// the normalisation reads (two bits per volume of the context):
 //   1. thresh_list_kernel  -- voxels in the band (two targets each: the voxel
 //                             and, on the kx = 0 plane, its SYMPLANE0 partner);
 //   2. hit_kernel          -- (target, section) pairs whose plane passes within

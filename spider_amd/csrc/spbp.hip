@@ -2,10 +2,11 @@
 // `BP 32F`) for MI355X (gfx950, CDNA4).  C ABI in include/spbp.h.
 //
 // Pipeline per chunk of B projections (all on one HIP stream):
-//   pad_kernel      PADD2 + ASTA_D (bp3f.f:1307-1343, asta.f:61-92): FP64 mean
-//                   outside the circle, zero-padded N x N image.
-//   hipFFT R2C      batched 2D forward transform (FMRS_2, fmrs_2.f:53); the
-//                   SPIDER sign (conjugate, fftw3.f:411-419) and the
+//   pad, rows       PADD2 + ASTA_D (bp3f.f:1307-1343, asta.f:61-92): FP64 mean
+//                   outside the circle; the nonzero rows' transforms.
+//   columns         the rest of the 2D forward transform (FMRS_2, fmrs_2.f:53;
+//                   hipFFT on padded images for N with other factors than 2,
+//                   3, 5 and 7); the SPIDER sign (conjugate, fftw3.f:411-419) and the
 //                   checkerboard (bp32f.f:859-864) are folded into the read of
 //                   the insertion kernel.
 //   insert kernel   ONELINE over every row J of every projection
@@ -13,13 +14,13 @@
 //                   bounds check, 5x5x5 Kaiser-Bessel scatter with reflected
 //                   taps, FP32 atomics into the half-grid X and weights W.
 // Finalisation per output volume:
-//   normalize       SYMPLANE0 (bp32f.f:1051-1088) evaluated on the fly, halves
+//   y pass          SYMPLANE0 (bp32f.f:1051-1088) evaluated on the fly, halves
 //                   summed (ADDADA, bp32f.f:345-346), X (-1)^(i+j+k) / W where
 //                   W > 0.1 (NRMW2, bp3f.f:1355-1366), FFTW c2r semantics on
 //                   the kx = 0 and kx = N/2 planes, conjugate (fftw3.f:430-437).
-//   hipFFT C2R      3D inverse (FMRS_3, fmrs_3.f:54).
-//   window          WINDKB2A (bp32f.f:945-1045): crop, x 1/N^3, divide by the
-//                   KB window transform, shell mean, sphere mask.
+//   z, x passes     3D inverse (FMRS_3, fmrs_3.f:54; hipFFT for those other N)
+//                   and WINDKB2A (bp32f.f:945-1045): crop, x 1/N^3, divide by
+//                   the KB window transform, shell mean, sphere mask.
 //
 // Accumulators stay raw (SYMPLANE0 is never applied in place), so inserts may
 // continue after a finalize and partial volumes merge linearly.
