@@ -78,7 +78,7 @@ __device__ inline float2 norm_val(const Acc& a, int nx, int N, int i, int j, int
 // The own inverse transform's blocks (inverse.hpp): 16 columns of N = 256 (8 of
 // 512).
 constexpr int INV_ELEMS = 4096, INV_NT = 512;
-constexpr int INV_LDS = INV_ELEMS + 96;   // columns are N + 1 apart; min(N / 2 + 1, INV_ELEMS / N) <= 65 of them
+constexpr int INV_LDS = INV_ELEMS + 96;   // columns are N + 1 apart; min(N / 2 + 1, INV_ELEMS / N) <= 46 of them
 inline int inv_slabs(int N) { const int cw = INV_ELEMS / N; return (N / 2 + 1 + cw - 1) / cw; }
 // Row pairs per block of the x pass: up to FFT_ROW_ELEMS values, but 256 blocks where the volume has them.
 inline int inv_pairs(int nx) {
