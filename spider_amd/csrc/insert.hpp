@@ -1,6 +1,7 @@
 // insert.hpp -- PADD2 and the ONELINE scatter kernels.
 #pragma once
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #include "common.hpp"
@@ -133,6 +134,29 @@ struct BrickGrid {
                          // cell (region = cells + 1 before and 2 after; insert_cells.hpp)
 };
 
+// brick shapes of the LDS-binned strategy (voxels; 3 x 8 B per voxel in LDS)
+// {x, y, z, owner-computes}; for owner-computes bricks the LDS region, whose
+// core (each sample's owner) is 4 voxels shorter per axis by nearest voxel
+// (1), 3 by unit cell (2)
+constexpr int NSHAPES = 8;
+constexpr int SHAPE_CELLS = 7, SHAPE_OWN = 8;   // unit cells; nearest voxel (not a plan of its own)
+constexpr int BRICK_SHAPES[NSHAPES + 1][4] = {{16, 16, 8, 0},  {16, 8, 8, 0},   {8, 8, 8, 0},
+                                              {16, 12, 8, 0},  {16, 16, 10, 0}, {16, 16, 12, 0},
+                                              {16, 16, 13, 0}, {12, 12, 12, 2}, {16, 16, 13, 1}};
+inline BrickGrid shape_grid(int nx, int shape) {
+    const int own = BRICK_SHAPES[shape][3], halo = own == 2 ? 3 : own ? 4 : 0;
+    BrickGrid g;
+    g.bx = BRICK_SHAPES[shape][0] - halo;
+    g.by = BRICK_SHAPES[shape][1] - halo;
+    g.bz = BRICK_SHAPES[shape][2] - halo;
+    g.own = own;
+    g.nbx = (nx + g.bx - 1) / g.bx;
+    g.nby = (2 * nx - 1 + g.by - 1) / g.by;
+    g.nbz = (2 * nx - 1 + g.bz - 1) / g.bz;
+    g.nb = g.nbx * g.nby * g.nbz;
+    return g;
+}
+
 __device__ inline void brick_origin(const BrickGrid& bg, int b, int nx, int& x0, int& y0, int& z0) {
     const int i = b % bg.nbx, j = (b / bg.nbx) % bg.nby, k = b / (bg.nbx * bg.nby);
     x0 = i * bg.bx;
@@ -166,6 +190,10 @@ inline size_t plane_hits(const BrickGrid& bg) {
                  cz = (size_t)bg.nbx * bg.nby * std::min(bg.nbz, (int)(len / bg.bz) + 1);
     return std::max(cx, std::max(cy, cz));
 }
+
+// The most sections of one launch: the lists' offsets and the work items'
+// (at most one per pair and one per key) are ints.
+inline size_t max_sections(const BrickGrid& bg) { return ((size_t)INT_MAX - 2 * (size_t)bg.nb) / plane_hits(bg); }
 
 // A section's plane (through the origin, normal n = DM(7:9)) feeds a brick
 // when it passes through the brick's expanded box and that box reaches into

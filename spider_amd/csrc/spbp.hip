@@ -62,15 +62,6 @@ namespace {
 // last failure messages: fixed buffers, so that no error path allocates
 constexpr int ERR_LEN = 512;
 thread_local char g_last_error[ERR_LEN] = {0};
-// brick shapes of the LDS-binned strategy (voxels; 3 x 8 B per voxel in LDS)
-// {x, y, z, owner-computes}; for owner-computes bricks the LDS region, whose
-// core (each sample's owner) is 4 voxels shorter per axis by nearest voxel
-// (1), 3 by unit cell (2)
-constexpr int NSHAPES = 8;
-constexpr int SHAPE_CELLS = 7, SHAPE_OWN = 8;   // unit cells; nearest voxel (not a plan of its own)
-constexpr int SHAPES[NSHAPES + 1][4] = {{16, 16, 8, 0},  {16, 8, 8, 0},   {8, 8, 8, 0},
-                                        {16, 12, 8, 0},  {16, 16, 10, 0}, {16, 16, 12, 0},
-                                        {16, 16, 13, 0}, {12, 12, 12, 2}, {16, 16, 13, 1}};
 // brick workgroups: 16x16x10, 16x16x12 and 16x16x13 (61.7, 73.8 and 80.2 KB of
 // LDS) run two 512-thread groups per CU; the others four (three for 16x16x8)
 // 256-thread groups.  The FP64-geometry instantiations need more VGPRs than
@@ -165,7 +156,7 @@ struct spbp_ctx {
     size_t hstage_cap = 0;
     // brick strategy
     int strategy = SPBP_STRAT_BRICK;
-    int shape = 3;   // index into SHAPES
+    int shape = 3;   // index into BRICK_SHAPES
     int C = 128;
     bool tuned = false;
     bool capturing = false;   // a batch graph is being captured: no host syncs, no timing events
@@ -332,18 +323,7 @@ int refuse_captured(spbp_ctx* c, const char* what) {
 // contexts have no shared-evaluation 16x16x12 / 16x16x13 kernels: 16x16x10).
 BrickGrid grid_of_shape(int nx, int flags, int& shape) {
     if ((flags & SPBP_GEOM_F64) && (shape == 5 || shape == 6)) shape = 4;
-    const int own = SHAPES[shape][3], halo = own == 2 ? 3 : own ? 4 : 0;
-    const int bx = SHAPES[shape][0] - halo, by = SHAPES[shape][1] - halo, bz = SHAPES[shape][2] - halo;
-    BrickGrid g;
-    g.bx = bx;
-    g.by = by;
-    g.bz = bz;
-    g.own = own;
-    g.nbx = (nx + bx - 1) / bx;
-    g.nby = (2 * nx - 1 + by - 1) / by;
-    g.nbz = (2 * nx - 1 + bz - 1) / bz;
-    g.nb = g.nbx * g.nby * g.nbz;
-    return g;
+    return shape_grid(nx, shape);
 }
 
 int configure_bricks(spbp_ctx* c, int shape) {
@@ -382,16 +362,26 @@ int configure_bricks(spbp_ctx* c, int shape) {
 // 256 172 / 138).
 bool few_sections(const spbp_ctx* c, int nsec) { return c->bgo.nb > 0 && nsec < 2 * c->nx * c->nvol; }
 
-// Projection lists for chunks of up to B projections.  The capacity is
+// The most images of one chunk whose sections' lists fit int offsets (0: not
+// even one image's); of either grid of the unit-cell shape.
+int list_images(const spbp_ctx* c) {
+    int shape = c->shape, so = SHAPE_OWN;
+    size_t n = max_sections(grid_of_shape(c->nx, c->flags, shape));
+    if (shape == SHAPE_CELLS) n = std::min(n, max_sections(grid_of_shape(c->nx, c->flags, so)));
+    return (int)std::min<size_t>(n / c->nsym, INT_MAX);
+}
+
+// Projection lists for launches of up to ns sections.  The capacity is
 // committed only once both arrays exist.
-int ensure_lists(spbp_ctx* c, int B) {
+int ensure_lists(spbp_ctx* c, size_t ns) {
     if (c->bg.nb <= 0) {   // an earlier allocation failed: the last good shape again
         const int rc = configure_bricks(c, c->shape);
         if (rc) return rc;
     }
-    // B images, nsym sections each, and the bricks a section hits at most (of either grid of the unit-cell shape)
-    const size_t cap = (size_t)B * c->nsym * std::max(plane_hits(c->bg), c->bgo.nb > 0 ? plane_hits(c->bgo) : 0);
-    const size_t ns = (size_t)B * c->nsym;
+    if (ns > max_sections(c->bg) || (c->bgo.nb > 0 && ns > max_sections(c->bgo)))
+        return fail(c, SPBP_ERR_ALLOC, "brick lists of %zu sections of %d^2 exceed 2^31 entries", ns, c->nx);
+    // the bricks a section hits at most (of either grid of the unit-cell shape)
+    const size_t cap = ns * std::max(plane_hits(c->bg), c->bgo.nb > 0 ? plane_hits(c->bgo) : 0);
     if (c->blist && c->bikey && c->blist_cap >= cap && c->bpln && c->bpln_cap >= ns) return SPBP_OK;
     if (c->graphs > 0) return refuse_captured(c, "growing the brick lists");
     c->blist_cap = 0;
@@ -408,12 +398,23 @@ int ensure_lists(spbp_ctx* c, int B) {
     return SPBP_OK;
 }
 
+// The lists of the committed chunk size after a change of shape or symmetry;
+// a chunk whose lists no longer fit is given up, and the next call makes a
+// smaller one.
+int refit_lists(spbp_ctx* c) {
+    if (c->fwd_batch > list_images(c)) c->fwd_batch = 0;
+    return c->fwd_batch > 0 ? ensure_lists(c, (size_t)c->fwd_batch * c->nsym) : SPBP_OK;
+}
+
 // Chunk buffers (and, for hipFFT transforms, the forward plan) for chunks of
-// want_batch projections.  c->fwd_batch is the committed chunk size: zero
-// until every buffer of the set exists.
+// want_batch projections, or as many as the brick lists can hold.
+// c->fwd_batch is the committed chunk size: zero until every buffer of the
+// set exists.
 int ensure_chunk(spbp_ctx* c, int want_batch) {
+    const int most = list_images(c), B = std::min(want_batch, most);
+    if (B < 1) return fail(c, SPBP_ERR_ALLOC, "brick lists of one image's %d sections of %d^2 exceed 2^31 entries", c->nsym, c->nx);
     const bool set = c->spec && c->vmax && (c->own_fwd() ? c->fmean != nullptr : (c->padbuf && c->fwd));
-    if (set && c->fwd_batch >= want_batch) return ensure_lists(c, c->fwd_batch);
+    if (set && c->fwd_batch >= B && c->fwd_batch <= most) return ensure_lists(c, (size_t)c->fwd_batch * c->nsym);
     if (c->graphs > 0) return refuse_captured(c, "growing the chunk buffers");
     c->fwd_batch = 0;
     if (c->padbuf) { (void)hipFree(c->padbuf); c->padbuf = nullptr; }
@@ -423,12 +424,12 @@ int ensure_chunk(spbp_ctx* c, int want_batch) {
     c->tail_batch = 0;
     if (c->vmax) { (void)hipFree(c->vmax); c->vmax = nullptr; }
     if (c->fmean) { (void)hipFree(c->fmean); c->fmean = nullptr; }
-    const int N = c->N, H = c->H, B = want_batch;
+    const int N = c->N, H = c->H;
     if (!c->own_fwd()) HIPCHK(c, dmalloc(&c->padbuf, (size_t)B * N * N * sizeof(float)));
     HIPCHK(c, dmalloc(&c->spec, (size_t)B * N * H * sizeof(float2)));
     HIPCHK(c, dmalloc(&c->vmax, (size_t)B * sizeof(float)));
     if (c->own_fwd()) HIPCHK(c, dmalloc(&c->fmean, (size_t)B * sizeof(double)));
-    int rc = ensure_lists(c, B);
+    int rc = ensure_lists(c, (size_t)B * c->nsym);
     if (rc) return rc;
     if (!c->own_fwd()) {   // own transforms need no plan, and the pad buffer is not used
         int n[2] = {N, N};
@@ -1185,7 +1186,7 @@ int apply_shape(spbp_ctx* c, int s) {
         for (int k = 1; k < NCVALS; ++k) if (c->tune_ms[s][k] < c->tune_ms[s][best]) best = k;
         c->C = CVALS[best];
     }
-    return c->fwd_batch > 0 ? ensure_lists(c, c->fwd_batch) : SPBP_OK;
+    return refit_lists(c);
 }
 
 // Time (ms, best of `reps`) one insertion plan over the b projections in
@@ -2024,7 +2025,7 @@ int spbp_tune(spbp_ctx* c, const void* imgs, int dtype, int nimg, const double* 
     }
     c->strategy = SPBP_STRAT_BRICK;
     for (int sh = 0; sh < NSHAPES && rc == SPBP_OK; ++sh) {
-        if ((rc = configure_bricks(c, sh)) || (rc = ensure_lists(c, c->fwd_batch))) break;
+        if ((rc = configure_bricks(c, sh)) || (rc = ensure_lists(c, (size_t)b * c->nsym))) break;
         for (int k = 0; k < NCVALS && rc == SPBP_OK; ++k) {
             c->C = CVALS[k];
             rc = time_plan(c, c->geom_d, b, t, st, 2, &ms);
@@ -2038,7 +2039,7 @@ int spbp_tune(spbp_ctx* c, const void* imgs, int dtype, int nimg, const double* 
         c->strategy = s_strat;
         c->C = s_C;
         (void)configure_bricks(c, s_shape);
-        (void)ensure_lists(c, c->fwd_batch);
+        (void)refit_lists(c);
         return rc;
     }
     int bs = 0, bk = 0;
@@ -2052,7 +2053,7 @@ int spbp_tune(spbp_ctx* c, const void* imgs, int dtype, int nimg, const double* 
     else if (c->tune_gather_ms < best_brick && c->tune_gather_ms < c->tune_direct_ms) c->strategy = SPBP_STRAT_GATHER;
     c->C = CVALS[bk];
     if ((rc = configure_bricks(c, bs))) return rc;
-    return ensure_lists(c, c->fwd_batch);
+    return refit_lists(c);
 }
 
 int spbp_get_plan(const spbp_ctx* c, int* strategy, int* shape, int* brick_proj, float* ms_per_proj) {
@@ -2080,7 +2081,7 @@ int spbp_set_plan(spbp_ctx* c, int strategy, int shape, int brick_proj) {
     if (brick_proj > 0) c->C = brick_proj;
     int rc = configure_bricks(c, shape);
     if (rc) return rc;
-    return c->fwd_batch > 0 ? ensure_lists(c, c->fwd_batch) : SPBP_OK;
+    return refit_lists(c);
 }
 
 }  // extern "C"
@@ -2715,7 +2716,7 @@ int spbp_set_symmetries(spbp_ctx* c, int nsym, const double* angles_deg) {
     c->smd = smd;
     c->nsym = nsym;
     c->tuned = false;
-    return c->fwd_batch > 0 ? ensure_lists(c, c->fwd_batch) : SPBP_OK;
+    return refit_lists(c);
 }
 
 int spbp_debug_fail_alloc(long k) {
