@@ -170,18 +170,20 @@ __device__ inline void brick_origin(const BrickGrid& bg, int b, int nx, int& x0,
 // product of DM(1:3) and DM(4:6), whose orthonormality the host has checked:
 // a unit vector whatever a caller's DM(7:9) holds, which bounds the bricks a
 // section can hit (plane_hits).
+__host__ __device__ inline float4 section_plane(const float* r, int half) {
+    return make_float4(r[1] * r[5] - r[2] * r[4], r[2] * r[3] - r[0] * r[5], r[0] * r[4] - r[1] * r[3], half ? 1.0f : 0.0f);
+}
 __global__ __launch_bounds__(TPB) void plane_pack_kernel(const Geom* __restrict__ geom, int n, float4* __restrict__ pln) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
-    const float* r = geom[p].r;
-    pln[p] = make_float4(r[1] * r[5] - r[2] * r[4], r[2] * r[3] - r[0] * r[5], r[0] * r[4] - r[1] * r[3],
-                         geom[p].half ? 1.0f : 0.0f);
+    if (p < n) pln[p] = section_plane(geom[p].r, geom[p].half);
 }
 
 // The most bricks one section's plane can hit: with n its unit normal and a
 // the axis of the largest |n|, the plane crosses a column of bricks along a
 // within |c_a - c*| <= h_a + h_b + h_c + 0.02 / |n_a| of the column's centre
 // line (h: half extents of the bricks' expanded boxes; |n_a| >= 1 / sqrt(3)).
+// brick_fill_kernel writes into buffers of this size unchecked: the CPU test
+// of the lists' sizes counts the hits of every shape against it.
 inline size_t plane_hits(const BrickGrid& bg) {
     const double mx = bg.own == 1 ? 2.52 : bg.own == 2 ? 0.52 : BRICK_MARGIN, m = bg.own ? 0.52 : BRICK_MARGIN;
     const double len = 2.0 * (0.5 * (bg.bx - 1) + mx + 0.5 * (bg.by - 1) + m + 0.5 * (bg.bz - 1) + m + 0.1);
@@ -195,7 +197,7 @@ inline size_t plane_hits(const BrickGrid& bg) {
 // (at most one per pair and one per key) are ints.
 inline size_t max_sections(const BrickGrid& bg) { return ((size_t)INT_MAX - 2 * (size_t)bg.nb) / plane_hits(bg); }
 
-// A section's plane (through the origin, normal n = DM(7:9)) feeds a brick
+// A section's plane (through the origin, normal n of section_plane) feeds a brick
 // when it passes through the brick's expanded box and that box reaches into
 // the sample disk of radius NX.  Owner-computes bricks expand their core by
 // 0.52 (samples whose nearest voxel lies in the core), and at kx = 0 by 2.52

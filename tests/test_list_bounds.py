@@ -1,5 +1,6 @@
 """The brick lists' sizes, on the CPU (tests/host/list_bounds.hip): the chunk
-limit keeps every list offset within an int."""
+limit keeps every list offset within an int, and no section hits more bricks
+than its buffer share."""
 import os
 import shutil
 import subprocess
