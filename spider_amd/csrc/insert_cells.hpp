@@ -15,10 +15,10 @@
 // bytes) in a pool in LDS and links it to its cell.  Then each lane takes up
 // to four samples of one cell and adds their terms for a tap in registers
 // before one LDS add.  The terms, their fixed-point encoding and so the sums
-// are insert_brick_kernel's (each term rounded once, the sums exact); the
-// weights' unit is 2^-48 instead of 2^-50, for the sum of four to fit.  The
-// table is in LDS too: as global loads its lookups, 64 scattered addresses
-// each, took the cache's tag rate (20.4 -> 18.8 ms, below).
+// are insert_brick_kernel's (each term rounded once, the weights to units of
+// 2^-WBITS, see CELL_WOFF; the sums exact).  The table is in LDS too: as
+// global loads its lookups, 64 scattered addresses each, took the cache's tag
+// rate (20.4 -> 18.8 ms, below).
 //
 // Measured against the nearest-voxel bricks, insertion per 20,000 images of
 // 128^2 (8 of 9 samples grouped by four, ~118 sections and ~5,900 samples per
@@ -48,11 +48,13 @@ constexpr int CELL_SECS = 120;    // sections of a work item at most
 constexpr int CELL_SECS64 = 96;   // with FP64 geometry
 constexpr int CELL_NT = 768;      // threads per workgroup, one workgroup per CU
 constexpr int CELL_EDGE = 9;      // cells per brick edge
-// Weight terms in units of 2^-48: a tap's sum over four samples (weights <= 1)
-// stays below 2^51, the range of the fused multiply-add encoding.
-constexpr int CELL_WBITS = 48;
-constexpr double CELL_WSCALE = 281474976710656.0;          // 2^48
-constexpr double CELL_WINV = 1.0 / 281474976710656.0;
+// Weights are positive, so a tap's sum over four samples is formed from 2^52
+// up, not from the middle of [2^52, 2^53) as signed terms are (fixed_term): at
+// four weights of exactly 1, the most it can be, it ends at 2^53, whose bit
+// pattern still is that of 2^52 plus the sum.
+constexpr double CELL_WOFF = 4503599627370496.0;                       // 2^52
+constexpr unsigned long long CELL_WOFF_BITS = 0x4330000000000000ull;   // its bits
+static_assert(4.0 * WSCALE <= 4503599627370496.0, "four weights of at most 1 stay within 2^52 units");
 
 __device__ __forceinline__ void add_global(Global<float> p, float v) {
     (void)__hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -188,7 +190,7 @@ __device__ __forceinline__ void cell_taps(Lds& L, const P (*g)[6], const unsigne
             for (int k = 0; k < K; ++k) tyz[k] = __fmul_rn(ty[k][ly], tz[k]);     // TY = TABI(Y) * TZ
 #pragma unroll
             for (int lx = 0; lx < 4; ++lx) {
-                double re = OFF, im = OFF, w = OFF;
+                double re = OFF, im = OFF, w = CELL_WOFF;
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
                     const double wd = (double)__fmul_rn(tx[k][lx], tyz[k]);       // WG = TABI(X) * TY
@@ -546,7 +548,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 256))) 
         const float* tab = L.tab;
         const P fltb = fltb_of<P>(J.fltb);
         const double vscale = ldexp(1.0, VBITS - e), vinv = ldexp(1.0, e - VBITS);
-        const double wscale = J.wscale * (CELL_WSCALE / WSCALE);   // a run-time value: kept in registers
+        const double wscale = J.wscale;   // a run-time value: kept in registers
         CellWalk wk;
         wk.s0 = wk.q0 = wk.total = wk.start = wk.cnt = 0;
         wk.lrec = wk.open = 0u;
@@ -632,9 +634,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 256))) 
             const size_t o = ((size_t)(kz >= 0 ? kz : N + kz) * N + (ky >= 0 ? ky : N + ky)) * H + kx;
             const long long tre = fixed_sum48(sre), tim = fixed_sum48(sim);
             if constexpr (WGT) {
-                const long long tw = (long long)(sw - (unsigned long long)fixed_count(sre, tre) * FIXED_OFF);
+                const long long tw = (long long)(sw - (unsigned long long)fixed_count(sre, tre) * CELL_WOFF_BITS);
                 if (tw == 0 && tre == 0 && tim == 0) continue;   // zero-weight taps only
-                const double wd = __dmul_rn((double)tw, CELL_WINV);
+                const double wd = __dmul_rn((double)tw, WINV);
                 const float wi = (float)wd;
                 if (Wc) twosum_atomic_add((float*)W, Wc, o, wi, (float)(wd - (double)wi));
                 else if (W) add_global(W + o, wi);
