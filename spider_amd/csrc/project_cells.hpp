@@ -7,22 +7,24 @@
 // samples of up to `C` sections whose planes cross the brick (the insertion's
 // lists and lattice walk), and every sample, one per lane, takes its taps
 // from LDS.  The region's layer kx = -1 holds conj X(1, -ky, -kz), so a
-// reflected tap is read like a direct one.  Taps and table lookups are the
-// insertion's; a row of four x taps is summed in FP64 and weighted by the
-// FP64 product of its y and z weights.
+// reflected tap is read like a direct one.  Taps, table lookups and the fp32
+// weights are the insertion's, as in gather_kernel; the products are summed
+// in FP64.  (A row of four x taps summed first and weighted by an unrounded
+// FP64 product took 3% less time, but transposed other weights than the
+// scatter's.)
 //
-// Measured, 2,048 sections of 128^2 (with lists and zero fill): 4.46 -> 1.38 ms;
-// 512 of 256^2 4.87 -> 1.58 ms.  It is bound by VALU issue (~570 per 64
-// samples: the walk 160, weights 100, taps 310) with the LDS reads (one
-// conflict-free 8-byte read per tap) at about half of that.
+// Measured, 2,048 sections of 128^2 (with lists and zero fill): 4.46 -> 1.42 ms;
+// 512 of 256^2 4.87 -> 1.63 ms.  It is bound by VALU issue (920 per 64
+// gathered samples) with the LDS reads (one conflict-free 8-byte read per
+// tap) at about half of that.
 #pragma once
 #include "common.hpp"
 #include "insert_cells.hpp"
 
 namespace spbp {
 
-constexpr int GATHER_NT = 256;      // 512 threads in two groups 1458 us per 2,048 of 128^2, 1966 per 512 of 256^2
-constexpr int GATHER_GROUPS = 4;    // workgroups per CU: 1375, 1576
+constexpr int GATHER_NT = 256;      // against four groups of 256, 512 threads in two took 6% more per 2,048 of 128^2, 25% per 512 of 256^2
+constexpr int GATHER_GROUPS = 4;    // workgroups per CU
 constexpr int GATHER_SECS = 128;    // sections of a work item at most
 
 template <typename P>
@@ -48,15 +50,14 @@ __device__ __forceinline__ f2v gather_taps(const GatherLds<P>& L, P x, P y, P z,
     // this lane's x and y taps in the cyclic order that gives the 16 lanes of a group distinct banks (own_taps)
     const int lane = threadIdx.x & 63;
     const int rx = (lane - xl) & 3, ry = ((lane >> 2) - yl) & 3;
-    double tx[4];
-    float ty[4], tz[4];
+    float tx[4], ty[4], tz[4];
     int xo[4], yo[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
         const int dx = (t + rx) & 3, dy = (t + ry) & 3;
         xo[t] = Lds::xpart(xl + dx);
         yo[t] = Lds::ypart(yl + dy) + Lds::zpart(zl);
-        tx[t] = (double)cell_weight(L.tab, x - (P)(x0 - 1 + xl + dx), fltb);
+        tx[t] = cell_weight(L.tab, x - (P)(x0 - 1 + xl + dx), fltb);
         ty[t] = cell_weight(L.tab, y - (P)(y0 - 1 + yl + dy), fltb);
         tz[t] = cell_weight(L.tab, z - (P)(z0 - 1 + zl + t), fltb);
     }
@@ -65,16 +66,14 @@ __device__ __forceinline__ f2v gather_taps(const GatherLds<P>& L, P x, P y, P z,
     for (int ly = 0; ly < 4; ++ly) {
 #pragma unroll
         for (int lz = 0; lz < 4; ++lz) {
-            double sr = 0.0, si = 0.0;
+            const float tyz = __fmul_rn(ty[ly], tz[lz]);               // TY = TABI(Y) * TZ
 #pragma unroll
             for (int lx = 0; lx < 4; ++lx) {
                 const f2v v = L.v[xo[lx] + yo[ly] + Lds::zpart(lz)];
-                sr = __fma_rn(tx[lx], (double)v.x, sr);
-                si = __fma_rn(tx[lx], (double)v.y, si);
+                const double w = (double)__fmul_rn(tx[lx], tyz);       // WG = TABI(X) * TY
+                re = __fma_rn(w, (double)v.x, re);
+                im = __fma_rn(w, (double)v.y, im);
             }
-            const double w = (double)ty[ly] * (double)tz[lz];
-            re = __fma_rn(w, sr, re);
-            im = __fma_rn(w, si, im);
         }
     }
     f2v o;

@@ -1,0 +1,58 @@
+"""GPU checks that the projector's gather carries ONELINE's own fp32 weights
+(TABI(X) * (TABI(Y) * TABI(Z)), each product rounded to fp32), whichever
+kernel a call's size takes: by bricks of unit cells or sample by sample.
+
+Both sum in FP64 and round once, so a value is within 2^-24 of itself of the
+oracle's FP64 sum over the same weights, and the two kernels are within one
+fp32 unit (2^-23) of each other; 2^-40 covers the FP64 sums (64 products of
+at most ~5, in any order).  Unrounded weights differ from these by up to
+2^-23 of a tap, which values smaller than their taps show.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from spider_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def grid(nx, rng):
+    N = 2 * nx
+    return (rng.standard_normal((N, N, nx + 1)) + 1j * rng.standard_normal((N, N, nx + 1))).astype(np.complex64)
+
+
+def parts(a):
+    return np.asarray(a, np.complex128).view(np.float64)
+
+
+# 2^19 pixels and more go by bricks; one case just below
+@pytest.mark.parametrize("nx,m", [(9, 6473), (16, 2048), (16, 2047), (33, 482), (75, 94)])
+def test_gather_carries_oneline_weights(nx, m):
+    from spider_amd import _lib, bp
+    rng = np.random.default_rng(200 + nx)
+    X = grid(nx, rng)
+    dm = _lib.rotations(synth.uniform_angles(m, rng)).reshape(m, 9)
+    print(f"case nx={nx} m={m}", flush=True)
+    with bp.Backprojector(nx) as b:
+        out = b.gather(torch.from_numpy(X).cuda(), dm=dm).cpu().numpy()
+    pick = np.unique(np.r_[0:24, rng.integers(0, m, 24), m - 1])
+    got, ref = parts(out[pick]), parts(oracle.gather(X.astype(np.complex128), dm[pick]))
+    assert np.all(np.abs(got - ref) <= 2.0**-24 * np.abs(ref) + 2.0**-40)
+
+
+@pytest.mark.parametrize("geom_f64", [False, True])
+@pytest.mark.parametrize("nx,m", [(10, 5243), (16, 2100), (40, 400)])
+def test_both_gathers_agree(nx, m, geom_f64):
+    from spider_amd import bp
+    rng = np.random.default_rng(300 + nx)
+    X = torch.from_numpy(grid(nx, rng)).cuda()
+    ang = synth.uniform_angles(m, rng)
+    print(f"case nx={nx} m={m} geom_f64={geom_f64}", flush=True)
+    with bp.Backprojector(nx, geom_f64=geom_f64) as b:
+        bricks = parts(b.gather(X, angles=ang).cpu().numpy())
+        samples = parts(np.concatenate([b.gather(X, angles=a).cpu().numpy() for a in np.array_split(ang, 3)]))
+    assert np.all(np.abs(bricks - samples) <= 2.0**-23 * np.abs(samples) + 2.0**-40)
+    assert np.any(samples != 0)
