@@ -728,9 +728,9 @@ int launch_bricks(spbp_ctx* c, const BrickJob* jh, int n, int* counter, hipStrea
     return launch_bricks_dev(c, c->jobs_d, n, counter, st, wgt, few);
 }
 
-// Per-(brick, half) projection lists of b projections (geometry at geom_d);
-// also zeroes c's queue head.
-int build_lists(spbp_ctx* c, const Geom* geom_d, int b, hipStream_t st, bool few) {
+// Per-(brick, half) projection lists of b projections (geometry at geom_d),
+// up to `per` to a work item; also zeroes c's queue head.
+int build_lists(spbp_ctx* c, const Geom* geom_d, int b, hipStream_t st, bool few, int per) {
     const BrickGrid& bg = few ? c->bgo : c->bg;
     if (c->bg.nb <= 0 || bg.nb > c->bg.nb || !c->bcnt || !c->blist || !c->bikey || c->blist_cap < (size_t)b * plane_hits(bg) || !c->bpln ||
         c->bpln_cap < (size_t)b)
@@ -743,7 +743,7 @@ int build_lists(spbp_ctx* c, const Geom* geom_d, int b, hipStream_t st, bool few
     plane_pack_kernel<<<nblocks(b), TPB, 0, st>>>(geom_d, b, c->bpln);
     brick_count_kernel<<<lgrid, TPB, 0, st>>>(c->bpln, b, bg, c->nx, c->bcnt);
     const int kb = (nkeys + 1023) / 1024;
-    key_scan_blocks_kernel<<<kb, 1024, 0, st>>>(c->bcnt, nkeys, item_proj(c->C, b, max_item(c, few)), c->boff, c->bioff, c->bscan);
+    key_scan_blocks_kernel<<<kb, 1024, 0, st>>>(c->bcnt, nkeys, per, c->boff, c->bioff, c->bscan);
     key_scan_sums_kernel<<<1, 1024, 0, st>>>(c->bscan, kb, nkeys, c->boff, c->bioff, c->bnext);
     key_scan_add_kernel<<<kb, 1024, 0, st>>>(nkeys, c->bscan, c->boff, c->bioff, c->bcur);
     brick_fill_kernel<<<lgrid, TPB, 0, st>>>(c->bpln, b, bg, c->nx, c->boff, c->bcur, c->blist);
@@ -805,7 +805,7 @@ int run_insert(spbp_ctx* c, int img0, const Geom* geom_d, int ng, const Targets&
         return fail(c, SPBP_ERR_ARG, "chunk buffers not allocated for %d sections", ng);
     if (own_kernel(c)) return launch_own(c, img0, geom_d, ng, t, st, units);
     const bool few = few_sections(c, ng);
-    int rc = build_lists(c, geom_d, ng, st, few);
+    int rc = build_lists(c, geom_d, ng, st, few, item_proj(c->C, ng, max_item(c, few)));
     if (rc) return rc;
     const BrickJob job = brick_job(c, img0, geom_d, ng, t, few);
     Timed tm(c, SPBP_K_INSERT, units, st);
@@ -895,13 +895,31 @@ int pad_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st) {
 // of unit cells where the context has their lists (the default shape) and the
 // launch enough samples, else sample by sample from memory.  A live batch
 // graph replays work on the lists, maybe on another stream: then, too, the
-// second.  The lists, the zero fill and the bricks' regions cost ~60 us and
-// more for larger grids: from NX sections and 2^19 pixels they are repaid
-// (by samples / by bricks, us: 64^2, 128 sections 103 / 102, 256 175 / 121;
-// 128^2, 128 314 / 247, 2048 4461 / 1425; 32^2, 100 38 / 65, 800 138 / 119;
-// 256^2, 256 2472 / 1519).
+// second.  The lists, the zero fill and the bricks' regions cost ~80 us and
+// more with the sections: repaid from NX sections and 2^19 pixels up, from
+// 2^20 where sample by sample runs out of an XCD's L2 with little of its 16 x
+// 16 tiles idle (NX 32 to 45; half grids of up to 3 MiB).  By samples / by
+// bricks, us: 9^2, 3236 sections 120 / 94; 16^2, 2048 186 / 113; 24^2, 910
+// 123 / 112; 32^2, 512 94 / 102, 1024 164 / 142; 36^2, 405 84 / 101, 809 139 /
+// 138; 44^2, 271 81 / 100, 542 134 / 132; 48^2, 228 122 / 100; 64^2, 128 99 /
+// 99, 256 176 / 126; 75^2, 93 92 / 102, 140 126 / 115; 128^2, 128 311 / 208,
+// 2048 4516 / 1413.
 bool gather_by_bricks(const spbp_ctx* c, int b) {
-    return c->shape == SHAPE_CELLS && c->graphs == 0 && b >= c->nx && (size_t)b * c->nx * c->nx >= (size_t)1 << 19;
+    const bool cached = c->nx >= 32 && c->nh * sizeof(float2) <= (size_t)3 << 20;
+    return c->shape == SHAPE_CELLS && c->graphs == 0 && b >= c->nx && (size_t)b * c->nx * c->nx >= (size_t)1 << (cached ? 20 : 19);
+}
+
+// Sections per work item of the gather: the plan's, halved (down to 16) while
+// the launch holds fewer than ~4 items per resident workgroup (plane_hits is
+// about four times a section's mean).  By the insertion's rule (one group per
+// CU: 8 items' sections) small boxes had too few items: 1966 sections of 20^2
+// 188 -> 131 us, 512 of 32^2 122 -> 102, 12945 of 9^2 197 -> 154; sample by
+// sample 207, 94 and 416.
+int gather_item(const spbp_ctx* c, int b) {
+    const size_t pairs = (size_t)b * plane_hits(c->bg), groups = (size_t)c->ncu * GATHER_GROUPS;
+    int k = std::min(c->C, GATHER_SECS);
+    while (k > 16 && pairs < 16 * groups * k) k >>= 1;
+    return k;
 }
 
 int launch_slices(spbp_ctx* c, const float2* X, const Geom* geom_d, int img0, int b, float2* out, hipStream_t st) {
@@ -911,7 +929,7 @@ int launch_slices(spbp_ctx* c, const float2* X, const Geom* geom_d, int img0, in
     if (gather_by_bricks(c, b) && c->blist && c->bikey && c->bpln_cap >= (size_t)b &&
         c->blist_cap >= (size_t)b * plane_hits(c->bg)) {
         fill((float*)out, 2 * (size_t)b * N * H, 0.0f, st);   // only samples are written
-        int rc = build_lists(c, geom_d, b, st, false);
+        int rc = build_lists(c, geom_d, b, st, false, gather_item(c, b));
         if (rc) return rc;
         const unsigned grid = (unsigned)c->ncu * GATHER_GROUPS;
         static_assert(GATHER_SECS >= CELL_SECS && GATHER_SECS >= CELL_SECS64, "the lists' items fit the gather's");
@@ -2188,7 +2206,7 @@ int enqueue_batch(const spbp_job* jobs, int njobs, Geom* const* geom, BrickJob* 
                 if ((rc = launch_own(c, p0, gj, b * c->nsym, t, st, b))) return rc;
                 continue;
             }
-            if ((rc = build_lists(c, gj, b * c->nsym, st, few))) return rc;
+            if ((rc = build_lists(c, gj, b * c->nsym, st, few, item_proj(c->C, b * c->nsym, max_item(c, few))))) return rc;
             units += b;
         }
         BrickJob table[MAX_JOBS];
@@ -3012,7 +3030,7 @@ int spbp_scatter_noalloc(int nx, int flags, const float* bi, int nimg, const dou
         const unsigned nbi = (unsigned)((N * H + BI_BLOCK - 1) / BI_BLOCK);
         bi_to_raw_kernel<<<nbi * b, TPB, 0, st>>>((const float2*)bi + (size_t)p0 * N * H, N, H, nbi, c.spec, c.vmax);
         HIPCHK(nullptr, hipGetLastError());
-        if ((rc = build_lists(&c, geom_d, b, st, false))) return fail(nullptr, rc, "%s", c.err);
+        if ((rc = build_lists(&c, geom_d, b, st, false, item_proj(c.C, b, max_item(&c, false))))) return fail(nullptr, rc, "%s", c.err);
         const BrickJob job = brick_job(&c, 0, geom_d, b, t, false);
         HIPCHK(nullptr, hipMemcpyAsync(job_d, &job, sizeof job, hipMemcpyHostToDevice, st));
         if ((rc = launch_bricks_dev(&c, job_d, 1, c.bnext, st, W != nullptr, false))) return fail(nullptr, rc, "%s", c.err);

@@ -28,8 +28,8 @@ def parts(a):
     return np.asarray(a, np.complex128).view(np.float64)
 
 
-# 2^19 pixels and more go by bricks; one case just below
-@pytest.mark.parametrize("nx,m", [(9, 6473), (16, 2048), (16, 2047), (33, 482), (75, 94)])
+# 2^19 pixels and more go by bricks (from 2^20 for NX 32 to 45); cases just below
+@pytest.mark.parametrize("nx,m", [(9, 6473), (16, 2048), (16, 2047), (33, 963), (33, 962), (75, 94)])
 def test_gather_carries_oneline_weights(nx, m):
     from spider_amd import _lib, bp
     rng = np.random.default_rng(200 + nx)
@@ -44,7 +44,7 @@ def test_gather_carries_oneline_weights(nx, m):
 
 
 @pytest.mark.parametrize("geom_f64", [False, True])
-@pytest.mark.parametrize("nx,m", [(10, 5243), (16, 2100), (40, 400)])
+@pytest.mark.parametrize("nx,m", [(10, 5243), (16, 2100), (40, 700)])
 def test_both_gathers_agree(nx, m, geom_f64):
     from spider_amd import bp
     rng = np.random.default_rng(300 + nx)
@@ -56,3 +56,19 @@ def test_both_gathers_agree(nx, m, geom_f64):
         samples = parts(np.concatenate([b.gather(X, angles=a).cpu().numpy() for a in np.array_split(ang, 3)]))
     assert np.all(np.abs(bricks - samples) <= 2.0**-23 * np.abs(samples) + 2.0**-40)
     assert np.any(samples != 0)
+
+
+@pytest.mark.parametrize("nx,m,bricks", [(16, 2048, True), (16, 2047, False), (31, 546, True), (32, 1024, True),
+                                         (32, 1023, False), (36, 405, False), (45, 518, True), (45, 517, False),
+                                         (46, 248, True), (75, 74, False)])
+def test_gather_route(nx, m, bricks):
+    """Where the bricks' lists and regions are not repaid a call goes sample by
+    sample: it builds no lists."""
+    from spider_amd import _lib, bp
+    rng = np.random.default_rng(400 + nx)
+    X = torch.from_numpy(grid(nx, rng)).cuda()
+    with bp.Backprojector(nx, timing=True) as b:
+        b.gather(X, angles=synth.uniform_angles(m, rng))
+        torch.cuda.synchronize()
+        assert b.kernel_stats(_lib.K_BIN)[1] == (1 if bricks else 0)
+        assert b.kernel_stats(_lib.K_GATHER)[1] == 1
