@@ -329,7 +329,8 @@ typedef struct {
 } spbp_job;
 /* Insert several jobs (distinct contexts, any box sizes, at most 64) as
  * spbp_insert would, with the scatter work of all of them in one persistent
- * kernel launch per round of chunks.  The contexts share one brick shape:
+ * kernel launch per round of chunks, or two where jobs with fewer than 2 NX
+ * sections per half and others meet.  The contexts share one brick shape:
  * the best total when all are tuned, else the first job's. */
 int spbp_insert_batch(const spbp_job* jobs, int njobs, void* stream);
 /* A batch captured as a HIP graph (pad, FFT, list build, persistent kernel;

@@ -2148,31 +2148,60 @@ int prepare_batch(const spbp_job* jobs, int njobs) {
     return SPBP_OK;
 }
 
-// Do the brick jobs of round r all hold few sections (one kernel serves them)?
-bool round_few(const spbp_job* jobs, int njobs, int r) {
-    for (int j = 0; j < njobs; ++j) {
-        const spbp_ctx* c = jobs[j].ctx;
-        const int p0 = r * c->fwd_batch;
-        if (p0 >= jobs[j].nimg || own_kernel(c)) continue;
-        if (!few_sections(c, std::min(c->fwd_batch, jobs[j].nimg - p0) * c->nsym)) return false;
-    }
-    return true;
+// Sections of job j's chunk in round r that go through a brick kernel (0: none left, or a kernel of its own).
+int round_sections(const spbp_job& j, int r) {
+    const spbp_ctx* c = j.ctx;
+    const int p0 = r * c->fwd_batch;
+    return p0 >= j.nimg || own_kernel(c) ? 0 : std::min(c->fwd_batch, j.nimg - p0) * c->nsym;
 }
 
+// Which jobs of a round take the nearest-voxel bricks: those with few sections
+// (few), those with more (many).  Each job its own way costs a second launch,
+// so a round splits only where that is repaid: a few-section job's cell items
+// cost ~25 us each, worth it from 2^20 pixels in all; the cells save ~30 us
+// per 2^20 pixels past the line, worth it from 2^22.  Below, one kernel
+// serves the round.  Graph replays, all by cells / all by nearest voxel / as
+// chosen here, us: 16 x 100 of 128^2 with 5,000: 12003 / 12748 / 10651; 4 x
+// 256 of 256^2 with 2,000: 21368 / 22191 / 18981; 100 of 128^2 with 3,000:
+// 3286 / 4405 / 3244; 8 x 40 of 32^2 with 3,000 of 128^2: 3247 / 4455 / 3247
+// (split 3280); 30 x 60 of 64^2 with 5 x 150: 3985 / 3600 / 3600 (split 3739);
+// 60 of 64^2 with 200: 325 / 310 / 310 (split 345).
+struct RoundRoute {
+    bool few = true, many = false;
+};
+RoundRoute round_route(const spbp_job* jobs, int njobs, int r) {
+    size_t small = 0, past = 0;
+    for (int j = 0; j < njobs; ++j) {
+        const spbp_ctx* c = jobs[j].ctx;
+        const int ng = round_sections(jobs[j], r);
+        const size_t npix = (size_t)c->nx * c->nx;
+        if (ng == 0) continue;
+        if (few_sections(c, ng)) small += npix * ng;
+        else past += npix * std::max(0, ng - 2 * c->nx * c->nvol);
+    }
+    RoundRoute t;
+    if (small == 0) return t;
+    if (small >= (size_t)1 << 20) t.many = past < (size_t)1 << 22;
+    else t.few = t.many = past < (size_t)1 << 20;
+    return t;
+}
+// Does job j of the round take the nearest-voxel bricks?
+bool nearest_voxel_job(const spbp_ctx* c, int ng, const RoundRoute& t) { return few_sections(c, ng) ? t.few : t.many && c->bgo.nb > 0; }
+
 // Host-side job table of round r: the brick jobs of the contexts that still
-// have a chunk in that round (direct- and gather-strategy contexts run their own kernels).
-// Depends only on device addresses, so it can be built before any work runs.
-int round_table(const spbp_job* jobs, int njobs, Geom* const* geom, int r, BrickJob* table, spbp_ctx** lead) {
+// have a chunk in that round (direct- and gather-strategy contexts run their
+// own kernels) and take the nearest-voxel bricks (few) or not.  Depends only
+// on device addresses, so it can be built before any work runs.
+int round_table(const spbp_job* jobs, int njobs, Geom* const* geom, int r, bool few, BrickJob* table, spbp_ctx** lead) {
     int n = 0;
-    const bool few = round_few(jobs, njobs, r);
+    const RoundRoute route = round_route(jobs, njobs, r);
     *lead = nullptr;
     for (int j = 0; j < njobs; ++j) {
         spbp_ctx* c = jobs[j].ctx;
-        const int p0 = r * c->fwd_batch;
-        if (p0 >= jobs[j].nimg || own_kernel(c)) continue;
+        const int p0 = r * c->fwd_batch, ng = round_sections(jobs[j], r);
+        if (ng == 0 || nearest_voxel_job(c, ng, route) != few) continue;
         const Targets t{c->X[0], c->W[0], c->X[1], c->W[1], c->Wc[0], c->Wc[1]};
-        const int b = std::min(c->fwd_batch, jobs[j].nimg - p0);
-        table[n++] = brick_job(c, p0, geom[j] + (size_t)p0 * c->nsym, b * c->nsym, t, few);
+        table[n++] = brick_job(c, p0, geom[j] + (size_t)p0 * c->nsym, ng, t, few);
         if (!*lead) *lead = c;   // its list build zeroes its queue head
     }
     return n;
@@ -2180,9 +2209,10 @@ int round_table(const spbp_job* jobs, int njobs, Geom* const* geom, int r, Brick
 
 // Enqueue the batch on st: per round, every job with projections left pads and
 // transforms its next chunk and builds its lists (or runs the direct kernel);
-// then one brick-kernel launch serves all jobs of the round.  geom[j] is job
-// j's device geometry.  With tables (graph capture), tables[r] must already
-// hold round r's job table in device memory: nothing is copied from the host.
+// then one brick-kernel launch serves the round, or one each the jobs with few
+// sections and the others (round_route).  geom[j] is job j's device geometry.  With
+// tables (graph capture), tables[2 r + few] must already hold round r's job
+// tables in device memory: nothing is copied from the host.
 int enqueue_batch(const spbp_job* jobs, int njobs, Geom* const* geom, BrickJob* const* tables, hipStream_t st) {
     int rounds = 0;
     for (int j = 0; j < njobs; ++j) {
@@ -2190,8 +2220,8 @@ int enqueue_batch(const spbp_job* jobs, int njobs, Geom* const* geom, BrickJob* 
         if (jobs[j].nimg > 0) rounds = std::max(rounds, (jobs[j].nimg + c->fwd_batch - 1) / c->fwd_batch);
     }
     for (int r = 0; r < rounds; ++r) {
-        const bool few = round_few(jobs, njobs, r);
-        long units = 0;
+        const RoundRoute route = round_route(jobs, njobs, r);
+        long units[2] = {0, 0};
         for (int j = 0; j < njobs; ++j) {
             spbp_ctx* c = jobs[j].ctx;
             const int p0 = r * c->fwd_batch;
@@ -2206,17 +2236,21 @@ int enqueue_batch(const spbp_job* jobs, int njobs, Geom* const* geom, BrickJob* 
                 if ((rc = launch_own(c, p0, gj, b * c->nsym, t, st, b))) return rc;
                 continue;
             }
-            if ((rc = build_lists(c, gj, b * c->nsym, st, few, item_proj(c->C, b * c->nsym, max_item(c, few))))) return rc;
-            units += b;
+            const int ng = b * c->nsym;
+            const bool few = nearest_voxel_job(c, ng, route);
+            if ((rc = build_lists(c, gj, ng, st, few, item_proj(c->C, ng, max_item(c, few))))) return rc;
+            units[few] += b;
         }
-        BrickJob table[MAX_JOBS];
-        spbp_ctx* lead = nullptr;
-        const int n = round_table(jobs, njobs, geom, r, table, &lead);
-        if (!n) continue;
-        Timed tm(lead, SPBP_K_INSERT, units, st);
-        const int rc = tables ? launch_bricks_dev(lead, tables[r], n, lead->bnext, st, true, few)
-                              : launch_bricks(lead, table, n, lead->bnext, st, true, few);
-        if (rc) return rc;
+        for (const bool few : {false, true}) {
+            BrickJob table[MAX_JOBS];
+            spbp_ctx* lead = nullptr;
+            const int n = round_table(jobs, njobs, geom, r, few, table, &lead);
+            if (!n) continue;
+            Timed tm(lead, SPBP_K_INSERT, units[few], st);
+            const int rc = tables ? launch_bricks_dev(lead, tables[2 * r + few], n, lead->bnext, st, true, few)
+                                  : launch_bricks(lead, table, n, lead->bnext, st, true, few);
+            if (rc) return rc;
+        }
     }
     return SPBP_OK;
 }
@@ -2249,7 +2283,7 @@ struct spbp_graph {
     std::vector<spbp_job> jobs;
     std::vector<std::vector<Geom>> hgeom;   // per job, the sections one launch inserts
     std::vector<Geom*> geom;          // per job, device (owned)
-    std::vector<BrickJob*> tables;    // per round, device (owned)
+    std::vector<BrickJob*> tables;    // per round and kernel (2 r + few), device (owned)
     hipStream_t stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -2334,17 +2368,17 @@ int spbp_graph_create(const spbp_job* jobs, int njobs, int reset_first, spbp_gra
             return bail(rc);
     }
     if (hipStreamSynchronize(g->stream) != hipSuccess) return bail(fail(nullptr, SPBP_ERR_DEVICE, "graph set-up"));
-    // every round's job table is uploaded now, synchronously: the captured
+    // every round's job tables are uploaded now, synchronously: the captured
     // work only reads these device copies
     const int rounds = batch_rounds(jobs, njobs);
-    g->tables.assign(rounds, nullptr);
-    for (int r = 0; r < rounds; ++r) {
+    g->tables.assign(2 * rounds, nullptr);
+    for (int k = 0; k < 2 * rounds; ++k) {
         BrickJob table[MAX_JOBS];
         spbp_ctx* lead = nullptr;
-        const int n = round_table(jobs, njobs, g->geom.data(), r, table, &lead);
+        const int n = round_table(jobs, njobs, g->geom.data(), k / 2, k % 2 != 0, table, &lead);
         if (!n) continue;
-        if (dmalloc(&g->tables[r], MAX_JOBS * sizeof(BrickJob)) != hipSuccess ||
-            hipMemcpy(g->tables[r], table, n * sizeof(BrickJob), hipMemcpyHostToDevice) != hipSuccess)
+        if (dmalloc(&g->tables[k], MAX_JOBS * sizeof(BrickJob)) != hipSuccess ||
+            hipMemcpy(g->tables[k], table, n * sizeof(BrickJob), hipMemcpyHostToDevice) != hipSuccess)
             return bail(fail(nullptr, SPBP_ERR_ALLOC, "graph job tables"));
     }
     for (int j = 0; j < njobs; ++j) jobs[j].ctx->capturing = true;
