@@ -300,11 +300,13 @@ int spbp_set_symmetries(spbp_ctx* ctx, int nsym, const double* angles_deg);
  * taps reach; 7, the default: owner-computes bins, each sample evaluated only
  * in the bin that holds its unit cell, a 12x12x12 LDS region around 9x9x9
  * cells -- or, in launches of fewer than 2 NX sections per half, its nearest
- * voxel, a 16x16x13 region around a 12x12x9 core) and projections per
- * brick work item (default 128; a launch of fewer than 8 x that many
- * sections halves it, down to 16, so its busiest bricks still split).  spbp_tune times every plan on a sample of
- * up to 1024 of the given images (into scratch grids: the accumulators are
- * untouched) and keeps the fastest; spbp_get_plan reports the plan and, when
+ * voxel, a 16x16x13 region around a 12x12x9 core) and projections per brick
+ * work item (default 128; a launch of fewer than 8 x that many sections halves
+ * it, down to 16, so its busiest bricks still split).  spbp_tune times every
+ * plan on a sample of up to 1024 of the given images, all in one half (into
+ * scratch grids: the accumulators are untouched), and keeps the fastest; plan
+ * 7 counts with the faster of its two kernels, whichever of them a launch of
+ * the sample's size would take.  spbp_get_plan reports the plan and, when
  * ms_per_proj is not NULL, the 34 measured ms per projection ([shape][C = 16,
  * 32, 64, 128], then direct, then gather).  The gather plan
  * (SPBP_STRAT_GATHER) is the scatter's transpose: each thread owns a voxel
