@@ -343,8 +343,9 @@ int spbp_insert_batch(const spbp_job* jobs, int njobs, void* stream);
  * would free or replace them fails with SPBP_ERR_ARG: spbp_destroy,
  * spbp_tune, spbp_set_symmetries, spbp_set_plan with another brick shape,
  * and insert / scatter / gather calls that need larger chunk buffers,
- * longer lists or a forward FFT plan for a new chunk size.  Calls that fit
- * the existing buffers may run between launches.  spbp_graph_launch replays
+ * longer lists or, where N is no power of two, a new partial chunk size (a
+ * forward FFT plan of its own in hipFFT's sizes).  Calls that fit the existing
+ * buffers may run between launches.  spbp_graph_launch replays
  * it on `stream`; spbp_graph_destroy releases the contexts. */
 typedef struct spbp_graph spbp_graph;
 int spbp_graph_create(const spbp_job* jobs, int njobs, int reset_first, spbp_graph** out);

@@ -442,13 +442,14 @@ int ensure_chunk(spbp_ctx* c, int want_batch) {
     return SPBP_OK;
 }
 
-// A partial chunk under a live batch graph: only the chunk size and the last
-// partial size set before are taken, whoever does the transforms.  (hipFFT
-// needs a plan per size; callers see one rule for every N that is no power of
-// two.)
+// A partial chunk under a live batch graph, for N that is no power of two: only
+// the chunk size and the last partial size run before are taken.  hipFFT's
+// sizes need a plan per size (plan_for); the own transforms need none, but
+// callers were promised one rule for all these N when hipFFT did them, and
+// what is refused stays refused.
 int tail_ok(spbp_ctx* c, int b) {
     if (b == c->fwd_batch || b == c->tail_batch) return SPBP_OK;
-    if (c->graphs > 0) return refuse_captured(c, "a new forward FFT plan");
+    if (c->graphs > 0) return refuse_captured(c, "a new partial chunk size");
     c->tail_batch = b;
     return SPBP_OK;
 }
