@@ -1890,9 +1890,15 @@ int spbp_gather(spbp_ctx* c, const float* X, int nimg, const double* angles_deg,
     hipStream_t st = (hipStream_t)stream;
     int rc = stage_geom(c, nimg, dm, angles_deg, nullptr, st, false);
     if (rc) return rc;
-    // the brick lists, where they can be had: without them the gather reads the grid sample by sample
-    const int B = std::min(c->batch, nimg);
-    if (gather_by_bricks(c, B) && ensure_lists(c, B) != SPBP_OK) (void)hipGetLastError();
+    // by bricks in chunks, whose lists are bounded; where those are too small for the bricks, or their lists cannot be
+    // had, all sections at once
+    int B = std::min(c->batch, nimg);
+    if (!gather_by_bricks(c, B)) {
+        B = nimg;
+    } else if (ensure_lists(c, B) != SPBP_OK) {
+        (void)hipGetLastError();
+        B = nimg;
+    }
     for (int p0 = 0; p0 < nimg; p0 += B) {
         const int b = std::min(B, nimg - p0);
         if ((rc = launch_slices(c, (const float2*)X, c->geom_d + p0, p0, b, (float2*)out_bi + (size_t)p0 * c->N * c->H, st)))

@@ -72,3 +72,19 @@ def test_gather_route(nx, m, bricks):
         torch.cuda.synchronize()
         assert b.kernel_stats(_lib.K_BIN)[1] == (1 if bricks else 0)
         assert b.kernel_stats(_lib.K_GATHER)[1] == 1
+
+
+@pytest.mark.parametrize("nx,m,batch,launches", [(16, 100, 16, 1), (16, 5000, 1024, 1), (16, 5000, 2048, 3), (16, 2100, 0, 1)])
+def test_gather_chunks(nx, m, batch, launches):
+    """A context's chunk size splits the gather where the chunks go by bricks;
+    sample by sample all sections go at once."""
+    from spider_amd import _lib, bp
+    rng = np.random.default_rng(500 + batch)
+    X = grid(nx, rng)
+    dm = _lib.rotations(synth.uniform_angles(m, rng)).reshape(m, 9)
+    with bp.Backprojector(nx, batch=batch, timing=True) as b:
+        out = b.gather(torch.from_numpy(X).cuda(), dm=dm).cpu().numpy()
+        assert b.kernel_stats(_lib.K_GATHER)[1] == launches
+    pick = np.unique(np.r_[0:20, rng.integers(0, m, 20), m - 1])
+    got, ref = parts(out[pick]), parts(oracle.gather(X.astype(np.complex128), dm[pick]))
+    assert np.all(np.abs(got - ref) <= 2.0**-24 * np.abs(ref) + 2.0**-40)
