@@ -114,6 +114,12 @@ int spbp_reset(spbp_ctx* ctx, void* stream);
  * out_bi: nimg x N x (NX+1) complex64 (device), ONELINE's BI layout (SPIDER
  * sign and checkerboard applied).  Rotations from angles_deg (host nimg x 3,
  * as spbp_insert) or, when dm is not NULL, dm (host nimg x 9 fp32).
+ * Calls of many sections (from NX sections and 2^19 pixels, 2^20 for NX 32 to
+ * 45) go by bricks on the default plan: they use the context's brick lists,
+ * growing them where they are too short (device memory, 8 bytes per section
+ * and brick its plane can hit: 110 MB for 4,096 sections of 128^2), and fall
+ * back to reading the grid sample by sample where that fails or a batch graph
+ * is live.
  * No counterpart in the reference: SPIDER's own projector PJ 3G
  * (pj3g.f:125) uses a different kernel; this is the projector whose adjoint
  * is BP 3F's insertion, for gradient and CG reconstruction. */

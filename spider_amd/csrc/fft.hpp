@@ -57,7 +57,7 @@ struct FftPlan {
     int N, np;
     int R[FFT_PASSES], Ns[FFT_PASSES];
     unsigned mNs[FFT_PASSES];   // by Ns
-    unsigned mN, mH, mL, mQ;    // by N, N / 2 + 1, N / 2 and N / 8 (0 for N < 16)
+    unsigned mH, mL, mQ;        // by N / 2 + 1, N / 2 and N / 8 (0 for N < 16)
 };
 __host__ __device__ inline unsigned recip(int d) { return d > 1 ? 0xFFFFFFFFu / (unsigned)d + 1 : 0; }
 __device__ __forceinline__ int div_by(int n, unsigned m) { return (int)__umulhi((unsigned)n, m); }   // d >= 2
@@ -67,7 +67,6 @@ inline FftPlan fft_plan(int N) {
     FftPlan p{};
     if (N < 8 || N > FFT_ROW_ELEMS || N % 2) return p;
     p.N = N;
-    p.mN = recip(N);
     p.mH = recip(N / 2 + 1);
     p.mL = recip(N / 2);
     p.mQ = N >= 16 ? recip(N / 8) : 0;

@@ -236,7 +236,7 @@ struct CellPoint {
 template <int CX, int CY, int CZ>
 struct CellLines {
     static constexpr double D2 = (CX + 0.04) * (CX + 0.04) + (CY + 0.04) * (CY + 0.04) + (CZ + 0.04) * (CZ + 0.04);
-    static constexpr int LINES = D2 <= 14 * 14 ? 16 : 21;
+    static constexpr int LINES = 21;
     static constexpr int WSEC = 64 / LINES;
     static_assert(D2 <= (LINES - 2) * (LINES - 2), "a section crosses at most the box diagonal + 2 lines");
 };

@@ -17,7 +17,8 @@
 // brick (ordered ballot compaction, 256 sections at a time), then every
 // thread tests each listed plane against its own voxel and, where it passes
 // within reach, walks the disc of candidate samples around t and -t
-// (for_candidates, shared with the NRMW2 re-summation).  Most candidates fail
+// (for_candidates; term_kernel of the NRMW2 re-summation lists the same
+// samples' bounding squares for its lanes instead).  Most candidates fail
 // the cheap window test, so the kernel does several times the arithmetic of
 // the scatter plans for the same terms; the tuner times it beside them.
 #pragma once

@@ -233,6 +233,8 @@ __device__ inline int sample_terms(const Geom& g, int I, int J, int nx, int N, c
 // Lattice samples that can reach t lie within 2.5 sqrt(3) of t or of -t in
 // the plane (in-plane coordinates (a, b) and (-a, -b)); visited rows J
 // ascending and I ascending within a row, as ONELINE's callers visit them.
+// The gather insertion's enumeration; term_kernel has its own (Runs), and a
+// sample either one adds carries no weight at t.
 template <typename P, typename F>
 __device__ inline void for_candidates(const Geom& g, int nx, int tx, int ty, int tz, F&& f) {
     const double a = (double)g.r[0] * tx + (double)g.r[1] * ty + (double)g.r[2] * tz;

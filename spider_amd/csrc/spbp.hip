@@ -128,7 +128,7 @@ struct spbp_ctx {
     int c2r_batch = 0, c2r2_batch = 0;
     float* c2rbuf = nullptr;
     int c2r_cap = 0;
-    // own forward transforms (power-of-two N): e^{-2 pi i m / N}, m < N
+    // own transforms (N = 2^a 3^b 5^c 7^d): e^{-2 pi i m / N}, m < N
     float2* tw = nullptr;
     FftPlan fft{};      // the own transforms' passes (N = 2^a 3^b 5^c 7^d), or np = 0: hipFFT's
     bool own_fwd() const { return fft.np > 0; }
@@ -847,8 +847,8 @@ int own_fft(spbp_ctx* c, const void* src, int dtype, int b, hipStream_t st, bool
         }
         {
             Timed tm(c, SPBP_K_FFT2, n, st);
-            const auto kernel = adjoint ? (c->pow2() ? col_fft_kernel<true, true> : col_fft_kernel<false, true>)
-                                        : (c->pow2() ? col_fft_kernel<true, false> : col_fft_kernel<false, false>);
+            // the adjoint's callers are held to powers of two (spbp_scatter_images)
+            const auto kernel = adjoint ? col_fft_kernel<true, true> : c->pow2() ? col_fft_kernel<true, false> : col_fft_kernel<false, false>;
             kernel<<<(unsigned)(n * slabs), FFT_COL_NT, lds, st>>>(c->nx, c->fft, slabs, width, c->tw, sp, c->vmax + s0);
         }
     }
