@@ -269,6 +269,8 @@ def run_throughput(args, config, nproj, steps, warmup, op="bp32f", bf16=False, t
     thresh = b.threshold_stats()
     b.close()
     opname = "BP 32F" if halves else "BP 3F"
+    # owner-computes plans take the kernel binned by unit cells (12x12x12 LDS regions) from 2 NX sections per half on
+    cells = bool(plan.get("owner_computes") and launches and units / launches >= 2 * nx * (2 if halves else 1))
     out = {"value": round(value, 2), "unit": "projections/s", "n_gpus": 1,
            "steps": steps, "warmup": warmup, "ms_per_step": round(dt / steps * 1e3, 3),
            "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
@@ -287,8 +289,8 @@ def run_throughput(args, config, nproj, steps, warmup, op="bp32f", bf16=False, t
                                      "finalize": round(fin_ms / steps, 3),
                                      "nrmw2_resum": round(res_ms / steps, 3)},
            "nrmw2_threshold": thresh,
-           "plan": {"strategy": plan["strategy"], "brick": list(plan["brick"]), "brick_proj": plan["brick_proj"],
-                    "owner_computes": plan.get("owner_computes", False),
+           "plan": {"strategy": plan["strategy"], "brick": [12, 12, 12] if cells else list(plan["brick"]),
+                    "brick_proj": plan["brick_proj"], "owner_computes": plan.get("owner_computes", False),
                     "tune_seconds": None if t_tune is None else round(t_tune, 3)}}
     if not extras:
         return out
@@ -300,8 +302,6 @@ def run_throughput(args, config, nproj, steps, warmup, op="bp32f", bf16=False, t
     avg_launch_s = ins_ms / 1e3 / launches
     per_launch = units / launches
     achieved = b_alg * per_launch / avg_launch_s / 1e9
-    # owner-computes plans take the kernel binned by unit cells from 2 NX sections per half on
-    cells = plan.get("owner_computes") and per_launch >= 2 * nx * (2 if halves else 1)
     kname = ("insert_direct_kernel" if plan["strategy"] == "direct"
              else "insert_cells_kernel<9,9,9>" if cells
              else "insert_brick_kernel<%d,%d,%d%s>" % (*plan["brick"], ",own" if plan.get("owner_computes") else ""))
